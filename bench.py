@@ -72,8 +72,11 @@ def no_gc():
 # (the autograd path's default) is the same stage as the plain backward.
 # the blend entry points, timed with HIP events inside the timed steps
 BLEND_ENTRIES = ("ubs_rasterize_to_pixels_fwd", "ubs_rasterize_to_pixels_fwd_prepacked", "ubs_rasterize_to_pixels_bwd",
-                 "ubs_rasterize_to_pixels_bwd_reuse")
+                 "ubs_rasterize_to_pixels_bwd_reuse", "ubs_rasterize_to_pixels_fwd_keep",
+                 "ubs_rasterize_to_pixels_bwd_keep")
 ENTRY_ALIASES = {"ubs_rasterize_to_pixels_bwd_reuse": "ubs_rasterize_to_pixels_bwd",
+                 "ubs_rasterize_to_pixels_bwd_keep": "ubs_rasterize_to_pixels_bwd",
+                 "ubs_rasterize_to_pixels_fwd_keep": "ubs_rasterize_to_pixels_fwd",
                  "ubs_rasterize_to_pixels_fwd_prepacked": "ubs_rasterize_to_pixels_fwd",
                  "ubs_beta_project_fwd_rec": "ubs_beta_project_fwd",
                  "ubs_isect_tiles_emit_ordered_cap": "ubs_isect_tiles_emit_ordered",
@@ -311,8 +314,7 @@ def blend_pair_stats(params, meta, img, tgt, W_: int, H_: int) -> dict:
                 "lane_evals_contributing": f[3], "entries_staged": f[4],
                 "in_support_frac": round(f[2] / max(f[1], 1), 4)},
         "bwd": {"wave_primitive_steps": b[0], "lane_evals_live": b[1], "lane_evals_contributing": b[2],
-                "reduce_scatter_steps": b[3], "entries_staged": b[4], "reduce_scatter_steps_le4_lanes": b[5],
-                "reduce_scatter_steps_le16_lanes": b[6],
+                "groups": b[3], "entries_tested": b[4], "plain_groups": b[5], "empty_group_slots": b[6],
                 "contributing_frac": round(b[2] / max(b[1], 1), 4)},
         "source": "counting builds of raster_fwd_kernel<16,3> / raster_bwd_kernel<16,3> (libubs_probe.so) on "
                   "this step's tile lists",

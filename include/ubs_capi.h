@@ -576,6 +576,23 @@ int ubs_rasterize_to_pixels_bwd_ckpt(uint32_t C, uint32_t N, int64_t n_isects, u
                                      float *v_opacities, float *v_betas, void *workspace,
                                      size_t workspace_bytes, void *stream);
 
+/* The blend forward as a training step runs it: ubs_rasterize_to_pixels_fwd,
+ * with the transmittance checkpoints of _fwd_ckpt when T_ckpt is not NULL and
+ * the prepacked records of _fwd_prepacked when prepacked is nonzero, that also
+ * keeps, when entry_masks is not NULL, which 8x8 sub-blocks of its tile every
+ * entry it reaches may touch (ubs_rasterize_entry_mask_bytes bytes), for
+ * ubs_rasterize_to_pixels_bwd_keep of the same inputs.  Same results. */
+size_t ubs_rasterize_entry_mask_bytes(int64_t n_isects, uint32_t tile_size);
+int ubs_rasterize_to_pixels_fwd_keep(uint32_t C, uint32_t N, int64_t n_isects, uint32_t channels,
+                                     const float *means2d, const float *conics, const float *colors,
+                                     const float *opacities, const float *betas, const float *backgrounds,
+                                     const uint8_t *masks, uint32_t width, uint32_t height, uint32_t tile_size,
+                                     uint32_t tile_width, uint32_t tile_height, const int32_t *tile_offsets,
+                                     const int32_t *flatten_ids, float *render_colors, float *render_alphas,
+                                     int32_t *last_ids, float *T_final, float *T_ckpt, size_t ckpt_floats,
+                                     int prepacked, void *entry_masks, size_t entry_mask_bytes, void *workspace,
+                                     size_t workspace_bytes, void *stream);
+
 /* ubs_rasterize_to_pixels_bwd (T_ckpt NULL) or _bwd_ckpt that reuses the
  * forward's packed primitive records and tile order instead of packing and
  * ordering again: fwd_workspace is the workspace the forward of the same
@@ -597,6 +614,22 @@ int ubs_rasterize_to_pixels_bwd_reuse(uint32_t C, uint32_t N, int64_t n_isects, 
                                       float *v_colors, float *v_opacities, float *v_betas,
                                       const void *fwd_workspace, size_t fwd_workspace_bytes, void *workspace,
                                       size_t workspace_bytes, void *stream);
+
+/* ubs_rasterize_to_pixels_bwd_reuse given the masks the forward kept
+ * (entry_masks NULL: the backward tests the entries itself).  Same results. */
+int ubs_rasterize_to_pixels_bwd_keep(uint32_t C, uint32_t N, int64_t n_isects, uint32_t channels,
+                                     const float *means2d, const float *conics, const float *colors,
+                                     const float *opacities, const float *betas, const float *backgrounds,
+                                     const uint8_t *masks, uint32_t width, uint32_t height, uint32_t tile_size,
+                                     uint32_t tile_width, uint32_t tile_height, const int32_t *tile_offsets,
+                                     const int32_t *flatten_ids, const float *render_alphas,
+                                     const int32_t *last_ids, const float *T_final, const float *T_ckpt,
+                                     size_t ckpt_floats, const float *v_render_colors,
+                                     const float *v_render_alphas, float *v_means2d, float *v_conics,
+                                     float *v_colors, float *v_opacities, float *v_betas, const void *entry_masks,
+                                     size_t entry_mask_bytes, const void *fwd_workspace,
+                                     size_t fwd_workspace_bytes, void *workspace, size_t workspace_bytes,
+                                     void *stream);
 
 /* ------------------------------------------------------------------------
  * Image loss of the training step: (1 - lambda) L1 + lambda (1 - SSIM).

@@ -213,8 +213,10 @@ static __global__ __launch_bounds__(kOrderThreads) void raster_block_order_kerne
 __device__ __forceinline__ void support_box(float a, float b, float c, float &hx, float &hy) {
     const float det = a * c - b * b;
     if (det > 0.f) {
-        hx = sqrtf(c / det) * 1.001f + 1e-3f;
-        hy = sqrtf(a / det) * 1.001f + 1e-3f;
+        // (hardware reciprocal and square root, 1 ulp each: far inside the padding)
+        const float inv = __builtin_amdgcn_rcpf(det);
+        hx = __builtin_amdgcn_sqrtf(c * inv) * 1.001f + 1e-3f;
+        hy = __builtin_amdgcn_sqrtf(a * inv) * 1.001f + 1e-3f;
     } else {
         hx = __builtin_huge_valf();
         hy = __builtin_huge_valf();
@@ -257,7 +259,13 @@ __host__ __device__ inline bool ellipse_meets_rect(float mx, float my, float a, 
     const float dy0 = my - hi_y, dy1 = my - lo_y;
     if (dx0 <= 0.f && dx1 >= 0.f && dy0 <= 0.f && dy1 >= 0.f) return true;
     if (!(a > 0.f && c > 0.f)) return true;
+#ifdef __HIP_DEVICE_COMPILE__
+    // only where on the edge the minimum is taken: 1 ulp there moves it by far
+    // less than the margin below
+    const float ia = __builtin_amdgcn_rcpf(a), ic = __builtin_amdgcn_rcpf(c);
+#else
     const float ia = 1.f / a, ic = 1.f / c;
+#endif
     float best = __builtin_huge_valf();
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
@@ -372,6 +380,25 @@ __host__ __device__ inline int64_t ckpt_slot(int32_t range_start, uint32_t tile_
 inline size_t ckpt_floats(uint32_t C, int64_t n_isects, uint32_t tw, uint32_t th, uint32_t tile_size) {
     const size_t BS = (size_t)tile_size * tile_size;
     return ((size_t)n_isects / BS + (size_t)C * tw * th + 1) * BS;
+}
+
+// Sub-block masks of the tile lists (optional): the forward's staging tests
+// every entry it reaches against the tile's 8x8 sub-blocks; kept per entry
+// (one byte, two for 32x32 tiles), they spare the backward the records and
+// tests of the entries that miss a sub-block.  Entries past the batch in which
+// the forward's tile was done are not written; no pixel's last contributor lies
+// there, so the backward reads none of them.
+template <int SB>
+struct EntryMask {
+    typedef uint8_t type;
+};
+template <>
+struct EntryMask<4> {
+    typedef uint16_t type;
+};
+
+inline size_t entry_mask_bytes(int64_t n_isects, uint32_t tile_size) {
+    return (size_t)n_isects * (tile_size == 32 ? 2 : 1);
 }
 
 // Channel chunks the kernels are instantiated for; wider colour vectors are

@@ -37,7 +37,8 @@ __global__ __launch_bounds__(TS *TS) void raster_fwd_kernel(
     float *__restrict__ render_colors, float *__restrict__ render_alphas, int32_t *__restrict__ last_ids,
     float *__restrict__ T_final, const float4 *__restrict__ rec, int wide_rec, float *__restrict__ T_ckpt,
     unsigned long long *__restrict__ stats = nullptr, const int64_t *__restrict__ n_dev = nullptr,
-    const uint32_t *__restrict__ order = nullptr, unsigned long long *__restrict__ wg_times = nullptr) {
+    const uint32_t *__restrict__ order = nullptr, unsigned long long *__restrict__ wg_times = nullptr,
+    void *__restrict__ entry_masks = nullptr) {
     // n_dev: the intersection count in device memory (at most n_isects, the
     // capacity of the lists), for callers that size the lists on the device
     if (n_dev) n_isects = min(max(*n_dev, (int64_t)0), n_isects);
@@ -147,7 +148,12 @@ __global__ __launch_bounds__(TS *TS) void raster_fwd_kernel(
             }
             float hx, hy;
             support_box(ca, cb, cc, hx, hy);
-            s_mask[tid] = g_ok ? subblock_mask_exact<SB>(xy.x, xy.y, ca, cb, cc, hx, hy, x0, y0) : 0u;
+            const uint32_t sub_mask = g_ok ? subblock_mask_exact<SB>(xy.x, xy.y, ca, cb, cc, hx, hy, x0, y0) : 0u;
+            s_mask[tid] = sub_mask;
+            if (entry_masks && write_meta) {  // for the backward
+                typedef typename EntryMask<SB>::type EM;
+                static_cast<EM *>(entry_masks)[batch_start + tid] = (EM)sub_mask;
+            }
         }
         __syncthreads();
         // ---- per-wave compaction of the batch to this sub-block's primitives
@@ -282,10 +288,11 @@ static int launch_fwd(uint32_t C, uint32_t N, int64_t n_isects, uint32_t channel
                       const float *betas, const float *bg, const uint8_t *masks, uint32_t W, uint32_t H,
                       uint32_t tw, uint32_t th, const int32_t *offs, const int32_t *flat, float *rc, float *ra,
                       int32_t *last, float *Tf, const float4 *rec, float *ck, const int64_t *n_dev,
-                      const uint32_t *order, hipStream_t st) {
+                      const uint32_t *order, void *em, hipStream_t st) {
     raster_fwd_kernel<TS, CDIM><<<xcd_grid(C, tw, th), TS * TS, 0, st>>>(
         C, N, n_isects, channels, coff, means2d, conics, colors, opac, betas, bg, masks, W, H, tw, th, offs, flat,
-        rc, ra, last, Tf, rec, rec && raster_wide_records(channels, TS) ? 1 : 0, ck, nullptr, n_dev, order);
+        rc, ra, last, Tf, rec, rec && raster_wide_records(channels, TS) ? 1 : 0, ck, nullptr, n_dev, order,
+        nullptr, em);
     UBS_LAUNCH_CHECK("raster_fwd_kernel");
     return UBS_OK;
 }
@@ -296,11 +303,11 @@ static int launch_fwd_chunk(int cd, uint32_t C, uint32_t N, int64_t n_isects, ui
                             const float *betas, const float *bg, const uint8_t *masks, uint32_t W, uint32_t H,
                             uint32_t tw, uint32_t th, const int32_t *offs, const int32_t *flat, float *rc,
                             float *ra, int32_t *last, float *Tf, const float4 *rec, float *ck, const int64_t *n_dev,
-                            const uint32_t *order, hipStream_t st) {
+                            const uint32_t *order, void *em, hipStream_t st) {
 #define UBS_FWD_CASE(K)                                                                                     \
     case K:                                                                                                 \
         return launch_fwd<TS, K>(C, N, n_isects, channels, coff, means2d, conics, colors, opac, betas, bg,  \
-                                 masks, W, H, tw, th, offs, flat, rc, ra, last, Tf, rec, ck, n_dev, order, st);
+                                 masks, W, H, tw, th, offs, flat, rc, ra, last, Tf, rec, ck, n_dev, order, em, st);
     switch (cd) {
         UBS_FWD_CASE(1)
         UBS_FWD_CASE(2)
@@ -309,17 +316,17 @@ static int launch_fwd_chunk(int cd, uint32_t C, uint32_t N, int64_t n_isects, ui
     case 8:
         if constexpr (TS <= 16)
             return launch_fwd<TS, 8>(C, N, n_isects, channels, coff, means2d, conics, colors, opac, betas, bg,
-                                     masks, W, H, tw, th, offs, flat, rc, ra, last, Tf, rec, ck, n_dev, order, st);
+                                     masks, W, H, tw, th, offs, flat, rc, ra, last, Tf, rec, ck, n_dev, order, em, st);
         break;
     case 16:
         if constexpr (TS <= 16)
             return launch_fwd<TS, 16>(C, N, n_isects, channels, coff, means2d, conics, colors, opac, betas, bg,
-                                      masks, W, H, tw, th, offs, flat, rc, ra, last, Tf, rec, ck, n_dev, order, st);
+                                      masks, W, H, tw, th, offs, flat, rc, ra, last, Tf, rec, ck, n_dev, order, em, st);
         break;
     case 32:
         if constexpr (TS <= 16)
             return launch_fwd<TS, 32>(C, N, n_isects, channels, coff, means2d, conics, colors, opac, betas, bg,
-                                      masks, W, H, tw, th, offs, flat, rc, ra, last, Tf, rec, ck, n_dev, order, st);
+                                      masks, W, H, tw, th, offs, flat, rc, ra, last, Tf, rec, ck, n_dev, order, em, st);
         break;
     default:
         break;
@@ -340,7 +347,7 @@ static int raster_fwd_impl(uint32_t C, uint32_t N, int64_t n_isects, uint32_t ch
                            const int32_t *flatten_ids, float *render_colors, float *render_alphas,
                            int32_t *last_ids, float *T_final, float *T_ckpt, size_t ckpt_n, void *workspace,
                            size_t workspace_bytes, void *stream, const int64_t *n_dev = nullptr,
-                           bool prepacked = false) {
+                           bool prepacked = false, void *entry_masks = nullptr) {
     hipStream_t st = as_stream(stream);
     UBS_REQUIRE(tile_size == 8 || tile_size == 16 || tile_size == 32, "tile_size must be 8, 16 or 32 (got %u)",
                 tile_size);
@@ -393,15 +400,18 @@ static int raster_fwd_impl(uint32_t C, uint32_t N, int64_t n_isects, uint32_t ch
         if (tile_size == 16)
             e = launch_fwd_chunk<16>(cd, C, N, n_isects, channels, coff, means2d, conics, colors, opacities, betas,
                                      backgrounds, masks, W, H, tw, th, tile_offsets, flatten_ids, render_colors,
-                                     render_alphas, last_ids, T_final, rec, T_ckpt, n_dev, order, st);
+                                     render_alphas, last_ids, T_final, rec, T_ckpt, n_dev, order,
+                                     entry_masks, st);
         else if (tile_size == 8)
             e = launch_fwd_chunk<8>(cd, C, N, n_isects, channels, coff, means2d, conics, colors, opacities, betas,
                                     backgrounds, masks, W, H, tw, th, tile_offsets, flatten_ids, render_colors,
-                                    render_alphas, last_ids, T_final, rec, T_ckpt, n_dev, order, st);
+                                    render_alphas, last_ids, T_final, rec, T_ckpt, n_dev, order,
+                                     entry_masks, st);
         else
             e = launch_fwd_chunk<32>(cd, C, N, n_isects, channels, coff, means2d, conics, colors, opacities, betas,
                                      backgrounds, masks, W, H, tw, th, tile_offsets, flatten_ids, render_colors,
-                                     render_alphas, last_ids, T_final, rec, T_ckpt, n_dev, order, st);
+                                     render_alphas, last_ids, T_final, rec, T_ckpt, n_dev, order,
+                                     entry_masks, st);
         if (e) return e;
         coff += (uint32_t)cd;
     }
@@ -461,6 +471,29 @@ extern "C" int ubs_rasterize_to_pixels_fwd_ckpt(uint32_t C, uint32_t N, int64_t 
     return raster_fwd_impl(C, N, n_isects, channels, means2d, conics, colors, opacities, betas, backgrounds, masks, W,
                            H, tile_size, tw, th, tile_offsets, flatten_ids, render_colors, render_alphas, last_ids,
                            T_final, T_ckpt, ckpt_n, workspace, workspace_bytes, stream);
+}
+
+extern "C" size_t ubs_rasterize_entry_mask_bytes(int64_t n_isects, uint32_t tile_size) {
+    return entry_mask_bytes(n_isects < 0 ? 0 : n_isects, tile_size);
+}
+
+extern "C" int ubs_rasterize_to_pixels_fwd_keep(
+    uint32_t C, uint32_t N, int64_t n_isects, uint32_t channels, const float *means2d, const float *conics,
+    const float *colors, const float *opacities, const float *betas, const float *backgrounds, const uint8_t *masks,
+    uint32_t W, uint32_t H, uint32_t tile_size, uint32_t tw, uint32_t th, const int32_t *tile_offsets,
+    const int32_t *flatten_ids, float *render_colors, float *render_alphas, int32_t *last_ids, float *T_final,
+    float *T_ckpt, size_t ckpt_n, int prepacked, void *entry_masks, size_t entry_mask_n, void *workspace,
+    size_t workspace_bytes, void *stream) {
+    UBS_REQUIRE(workspace || !prepacked, "prepacked records need the workspace that holds them");
+    UBS_REQUIRE(n_isects >= 0, "n_isects out of range");
+    if (entry_masks && entry_mask_n < entry_mask_bytes(n_isects, tile_size)) {
+        set_error("entry masks of %zu bytes, %zu needed", entry_mask_n, entry_mask_bytes(n_isects, tile_size));
+        return UBS_ERR_WORKSPACE;
+    }
+    return raster_fwd_impl(C, N, n_isects, channels, means2d, conics, colors, opacities, betas, backgrounds, masks, W,
+                           H, tile_size, tw, th, tile_offsets, flatten_ids, render_colors, render_alphas, last_ids,
+                           T_final, T_ckpt, ckpt_n, workspace, workspace_bytes, stream, nullptr, prepacked != 0,
+                           entry_masks);
 }
 
 extern "C" size_t ubs_transmittance_checkpoint_floats(uint32_t C, int64_t n_isects, uint32_t tile_width,

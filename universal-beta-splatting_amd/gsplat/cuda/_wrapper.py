@@ -672,10 +672,12 @@ def raster_fwd_ckpt_raw(means2d, conics, colors, opacities, betas, backgrounds, 
 
 
 def _raster_fwd(means2d, conics, colors, opacities, betas, backgrounds, masks, width, height, tile_size,
-                isect_offsets, flatten_ids, checkpoint: bool, prepacked=None):
+                isect_offsets, flatten_ids, checkpoint: bool, prepacked=None, keep_masks: bool = False):
     """(render_colors, render_alphas, last_ids, T_final, T_ckpt or None, the
     workspace: None, or the packed records and, with the tile order on, the
-    order, which the backward of the same inputs can reuse)."""
+    order, which the backward of the same inputs can reuse); with keep_masks
+    also the sub-block masks of the entries, for that backward (None without
+    a workspace)."""
     require_cuda(means2d, conics, colors, opacities, betas, backgrounds, isect_offsets, flatten_ids)
     require_dtype(_F32, means2d, conics, colors, opacities, betas, backgrounds)
     require_dtype(_I32, isect_offsets, flatten_ids)
@@ -693,29 +695,35 @@ def _raster_fwd(means2d, conics, colors, opacities, betas, backgrounds, masks, w
     else:
         prepacked = None
         ws, ws_bytes = _blend_workspace(C, N, False, dev, tw, th)
-    if not checkpoint:
+    n = flatten_ids.numel()
+    common = (C, N, n, channels, ptr(means2d), ptr(conics), ptr(colors), ptr(opacities), ptr(betas),
+              ptr(backgrounds), mp[0] if mp else None, width, height, tile_size, tw, th, ptr(isect_offsets),
+              ptr(flatten_ids), ptr(render_colors), ptr(render_alphas), ptr(last_ids), ptr(T_final))
+    st = stream_of(means2d)
+    T_ckpt = emasks = None
+    if checkpoint:
+        n_ck = int(lib().ubs_transmittance_checkpoint_floats(C, n, tw, th, tile_size))
+        T_ckpt = torch.empty((n_ck,), dtype=torch.float32, device=dev)
+    if keep_masks and ws is not None:
+        emasks = torch.empty((n * (2 if tile_size == 32 else 1),), dtype=torch.uint8, device=dev)
+        _call("ubs_rasterize_to_pixels_fwd_keep", *common, ptr(T_ckpt), 0 if T_ckpt is None else T_ckpt.numel(),
+              0 if prepacked is None else 1, ptr(emasks), emasks.numel(), ptr(ws), ws_bytes, st)
+    elif checkpoint:
+        _call("ubs_rasterize_to_pixels_fwd_ckpt", *common, ptr(T_ckpt), n_ck, ptr(ws), ws_bytes, st)
+    else:
         entry = "ubs_rasterize_to_pixels_fwd_prepacked" if prepacked is not None else "ubs_rasterize_to_pixels_fwd"
-        _call(entry, C, N, flatten_ids.numel(), channels, ptr(means2d), ptr(conics),
-              ptr(colors), ptr(opacities), ptr(betas), ptr(backgrounds), mp[0] if mp else None, width, height,
-              tile_size, tw, th, ptr(isect_offsets), ptr(flatten_ids), ptr(render_colors), ptr(render_alphas),
-              ptr(last_ids), ptr(T_final), ptr(ws), ws_bytes, stream_of(means2d))
-        return render_colors, render_alphas, last_ids, T_final, None, ws
-    n_ck = int(lib().ubs_transmittance_checkpoint_floats(C, flatten_ids.numel(), tw, th, tile_size))
-    T_ckpt = torch.empty((n_ck,), dtype=torch.float32, device=dev)
-    _call("ubs_rasterize_to_pixels_fwd_ckpt", C, N, flatten_ids.numel(), channels, ptr(means2d), ptr(conics),
-          ptr(colors), ptr(opacities), ptr(betas), ptr(backgrounds), mp[0] if mp else None, width, height,
-          tile_size, tw, th, ptr(isect_offsets), ptr(flatten_ids), ptr(render_colors), ptr(render_alphas),
-          ptr(last_ids), ptr(T_final), ptr(T_ckpt), n_ck, ptr(ws), ws_bytes, stream_of(means2d))
-    return render_colors, render_alphas, last_ids, T_final, T_ckpt, ws
+        _call(entry, *common, ptr(ws), ws_bytes, st)
+    out = (render_colors, render_alphas, last_ids, T_final, T_ckpt, ws)
+    return (*out, emasks) if keep_masks else out
 
 
 def raster_bwd_raw(means2d, conics, colors, opacities, betas, backgrounds, masks, width, height, tile_size,
                    isect_offsets, flatten_ids, render_alphas, last_ids, T_final, v_render_colors,
-                   v_render_alphas, T_ckpt=None, fwd_workspace=None):
+                   v_render_alphas, T_ckpt=None, fwd_workspace=None, entry_masks=None):
     """Blend backward.  fwd_workspace: the workspace the forward of the same
     inputs returned (records and tile order, sized with the order): its
     records and order are reused (ubs_rasterize_to_pixels_bwd_reuse) instead
-    of packed and computed again."""
+    of packed and computed again; entry_masks: the masks that forward kept."""
     require_cuda(means2d, conics, colors, opacities, betas, backgrounds, isect_offsets, flatten_ids,
                  render_alphas, last_ids, T_final, v_render_colors, v_render_alphas)
     require_dtype(_F32, means2d, conics, colors, opacities, betas, backgrounds, render_alphas, T_final,
@@ -736,12 +744,15 @@ def raster_bwd_raw(means2d, conics, colors, opacities, betas, backgrounds, masks
             require_dtype(_F32, T_ckpt)
         gb = int(lib().ubs_rasterize_workspace_bytes(C, N, 0))
         gws = torch.empty((gb,), dtype=torch.uint8, device=means2d.device)
-        _call("ubs_rasterize_to_pixels_bwd_reuse", C, N, flatten_ids.numel(), channels, ptr(means2d), ptr(conics),
+        if entry_masks is not None:
+            require_cuda(entry_masks)
+        _call("ubs_rasterize_to_pixels_bwd_keep", C, N, flatten_ids.numel(), channels, ptr(means2d), ptr(conics),
               ptr(colors), ptr(opacities), ptr(betas), ptr(backgrounds), mp[0] if mp else None, width, height,
               tile_size, tw, th, ptr(isect_offsets), ptr(flatten_ids), ptr(render_alphas), ptr(last_ids),
               ptr(T_final), ptr(T_ckpt), 0 if T_ckpt is None else T_ckpt.numel(), ptr(v_render_colors),
               ptr(v_render_alphas), ptr(v_means2d), ptr(v_conics), ptr(v_colors), ptr(v_opacities), ptr(v_betas),
-              ptr(fwd_workspace), fwd_workspace.numel(), ptr(gws), gb, stream_of(means2d))
+              ptr(entry_masks), 0 if entry_masks is None else entry_masks.numel(), ptr(fwd_workspace),
+              fwd_workspace.numel(), ptr(gws), gb, stream_of(means2d))
         return v_means2d, v_conics, v_colors, v_opacities, v_betas
     ws, ws_bytes = _blend_workspace(C, N, True, means2d.device, tw, th)
     if T_ckpt is None:
@@ -1141,14 +1152,16 @@ class _RasterizeToPixels(torch.autograd.Function):
         ckpt = _t_checkpoint and any(ctx.needs_input_grad[:5])
         # an output without a gradient comes back as None, not a filled zero tensor
         ctx.set_materialize_grads(False)
-        render_colors, render_alphas, last_ids, T_final, T_ckpt, ws = _raster_fwd(
+        grad = any(ctx.needs_input_grad[:5])
+        render_colors, render_alphas, last_ids, T_final, T_ckpt, ws, *emasks = _raster_fwd(
             means2d, conics, colors, opacities, betas, backgrounds, masks, width, height, tile_size,
-            isect_offsets, flatten_ids, ckpt, prepacked)
+            isect_offsets, flatten_ids, ckpt, prepacked, keep_masks=grad and _tile_order)
         ctx.save_for_backward(means2d, conics, colors, opacities, betas, backgrounds, masks, isect_offsets,
                               flatten_ids, render_alphas, last_ids, T_final, T_ckpt)
         ctx.width, ctx.height, ctx.tile_size = width, height, tile_size
         # the forward's packed records and tile order, for the backward to reuse
-        ctx.fwd_ws = ws if (ws is not None and _tile_order and any(ctx.needs_input_grad[:5])) else None
+        ctx.fwd_ws = ws if (ws is not None and _tile_order and grad) else None
+        ctx.emasks = emasks[0] if emasks else None
         return render_colors, render_alphas
 
     @staticmethod
@@ -1162,8 +1175,8 @@ class _RasterizeToPixels(torch.autograd.Function):
             means2d, conics, colors, opacities, betas, backgrounds, masks, ctx.width, ctx.height,
             ctx.tile_size, isect_offsets, flatten_ids, render_alphas, last_ids, T_final,
             v_render_colors.contiguous(), None if v_render_alphas is None else v_render_alphas.contiguous(),
-            T_ckpt=T_ckpt, fwd_workspace=ctx.fwd_ws)
-        ctx.fwd_ws = None
+            T_ckpt=T_ckpt, fwd_workspace=ctx.fwd_ws, entry_masks=ctx.emasks)
+        ctx.fwd_ws = ctx.emasks = None
         if ctx.needs_input_grad[5]:
             v_backgrounds = (v_render_colors * (1.0 - render_alphas).float()).sum(dim=(1, 2))
         else:
