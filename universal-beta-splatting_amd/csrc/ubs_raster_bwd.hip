@@ -147,10 +147,6 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Largest opacity for which alpha cannot reach the 0.999 clamp
-// ((1 - sigma)^beta <= 1 up to a few ulp for beta >= 0).
-constexpr float kNoClampOpacity = 0.998f;
-
 // STATS (measurement builds only; the library's kernels have it off) counts
 // into stats[0..6]: (wave, primitive) evaluations, lane evaluations at or
 // before the pixel's last contributor, of those that contribute, groups of 16

@@ -4,21 +4,30 @@
 // pixel sub-block of the tile (lane l -> pixel (l & 7, l >> 3) of it), which
 // is the unit of culling: a batch of TS*TS primitives is staged in LDS, every
 // primitive gets a bit mask of the sub-blocks its sigma < 1 ellipse reaches
-// (bounding-box test refined by an exact ellipse/rectangle test), and each
+// (bounding-box test refined by an ellipse/rectangle test), and each
 // wave compacts the batch to the primitives that touch its sub-block (ballot
 // + popcount) before the per-pixel front-to-back loop.
 // Pixels stop at the first primitive that would take transmittance to
 // <= 1e-4 (exclusive), as rasterize_to_pixels_fwd.cu:150-172 does; a wave
 // leaves the batch as soon as all of its pixels are done and the workgroup
 // stops loading batches once every pixel is done.
+//
+// Bound by VALU issue: 24 instructions per (wave, primitive) step, two of them
+// quarter-rate (log2, exp2), ~75 SIMD cycles in all; at 1080p / 1M primitives
+// the 20.7 M steps are 0.66 ms of the 0.75 ms measured (0.98 ms before the steps
+// below), the rest staging.  Next to it the loop's LDS reads (42 bytes a step,
+// 11.7 cycles per CU) take 0.41 ms.
 #pragma clang fp contract(off)
+
+#include <type_traits>
 
 #include "ubs_raster.h"
 
-// Read two compacted-list entries and both their records before blending
-// either (1), or one entry at a time (0).
-#ifndef UBS_FWD_PAIRED_READS
-#define UBS_FWD_PAIRED_READS 1
+// Primitives per step of the blend loop (a power of two).  1080p / 1M: 2 takes
+// 750 us at 6-7 waves per SIMD, 4 815 us (98 VGPRs), 8 900 us (146 VGPRs); 4 held
+// to 72 VGPRs spills and takes 762 us.
+#ifndef UBS_FWD_STEP
+#define UBS_FWD_STEP 2
 #endif
 
 namespace ubs {
@@ -45,13 +54,16 @@ __global__ __launch_bounds__(TS *TS) void raster_fwd_kernel(
     constexpr int BS = TS * TS;        // threads = batch size
     constexpr int SB = TS / 8;         // sub-blocks per tile side
     constexpr int NW = BS / 64;        // waves
-    __shared__ float4 s_geo[BS];       // x, y, a, 2b
-    __shared__ float4 s_geo2[BS];      // c, opacity, beta, (unused)
-    // up to 4 channels: one float4 per primitive, addressed with the same
-    // byte offset as s_geo / s_geo2 (no per-primitive address arithmetic)
+    // (slot BS: an entry that contributes nowhere, for the odd end of a list)
+    __shared__ float4 s_geo[BS + 1];   // x, y, a, 2b
+    __shared__ float4 s_geo2[BS + 1];  // c, opacity, beta, first colour
+    // up to 4 channels: the first beside the geometry, the others in a float4 per
+    // primitive, addressed with the same byte offset as s_geo / s_geo2 (no
+    // per-primitive address arithmetic) and read as the 4, 8 or 16 bytes that
+    // are in use: the loop's broadcast reads share the CU's LDS bandwidth
     constexpr bool kColVec = CDIM <= 4;
-    __shared__ float4 s_colv[kColVec ? BS : 1];
-    __shared__ float s_col[kColVec ? 1 : CDIM][kColVec ? 1 : BS];
+    __shared__ float4 s_colv[kColVec && CDIM > 1 ? BS + 1 : 1];
+    __shared__ float s_col[kColVec ? 1 : CDIM][kColVec ? 1 : BS + 1];
     __shared__ uint32_t s_mask[BS];
     // byte offsets (16 x entry) of the wave's primitives; 32-bit so that a
     // pair of them is one 64-bit read with nothing to unpack
@@ -97,25 +109,41 @@ __global__ __launch_bounds__(TS *TS) void raster_fwd_kernel(
     const float px = (float)j + 0.5f, py = (float)i + 0.5f;
     const float x0 = (float)(tx * TS), y0 = (float)(ty * TS);
 
+    if (tid == 0) {
+        s_geo[BS] = make_float4(__builtin_huge_valf(), 0.f, 0.f, 0.f);
+        s_geo2[BS] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (!kColVec) {
+#pragma unroll
+            for (int k = 0; k < CDIM; ++k) s_col[k][BS] = 0.f;
+        } else if constexpr (CDIM > 1) {
+            s_colv[BS] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
     float T = 1.f;
     int32_t cur = 0;
-    bool done = !inside;
+    // the pixel centre's x, NaN once the pixel is done: its sigma is then NaN
+    // and no primitive contributes
+    float bx = inside ? px : __builtin_nanf("");
     float acc[CDIM];
 #pragma unroll
     for (int k = 0; k < CDIM; ++k) acc[k] = 0.f;
 
     uint32_t st_steps = 0, st_live = 0, st_sup = 0, st_take = 0, st_staged = 0;
+    int32_t g_next = range_start + tid < range_end ? flatten_ids[range_start + tid] : 0;  // of the next batch
     const int32_t nb = range_end > range_start ? (range_end - range_start + BS - 1) / BS : 0;
     for (int32_t b = 0; b < nb; ++b) {
-        if (__syncthreads_count(done) >= BS) break;
+        if (__syncthreads_count(bx != bx) >= BS) break;
         const int32_t batch_start = range_start + b * BS;
         const int32_t cnt = min(BS, range_end - batch_start);
         if constexpr (STATS) st_staged += (uint32_t)(tid < cnt);
-        // ---- stage one primitive per thread
+        // ---- stage one primitive per thread (its id was loaded a batch ahead: the
+        // record's address does not wait for it)
+        const int32_t g_raw = g_next;
+        if (batch_start + BS + tid < range_end) g_next = flatten_ids[batch_start + BS + tid];
+        uint32_t staged_mask = 0;
         if (tid < cnt) {
             // an id outside [0, C N) (only from a sort that gave up) stages
             // primitive 0 with an empty sub-block mask: never blended
-            const int32_t g_raw = flatten_ids[batch_start + tid];
             const bool g_ok = (uint64_t)(uint32_t)g_raw < (uint64_t)C * N;
             const int32_t g = g_ok ? g_raw : 0;
             float2 xy;
@@ -136,48 +164,188 @@ __global__ __launch_bounds__(TS *TS) void raster_fwd_kernel(
                 op = opacities[g]; be = betas[g];
             }
             s_geo[tid] = make_float4(xy.x, xy.y, ca, 2.f * cb);
-            s_geo2[tid] = make_float4(cc, op, be, 0.f);
             const float *cp = colors + (int64_t)g * channels + coff;
             if constexpr (kColVec) {
-                s_colv[tid] = (rec && wide_rec) ? cw
-                                                : make_float4(cp[0], CDIM > 1 ? cp[1] : 0.f, CDIM > 2 ? cp[2] : 0.f,
-                                                              CDIM > 3 ? cp[3] : 0.f);
-            } else {
+                if (!(rec && wide_rec))
+                    cw = make_float4(cp[0], CDIM > 1 ? cp[1] : 0.f, CDIM > 2 ? cp[2] : 0.f, CDIM > 3 ? cp[3] : 0.f);
+                if constexpr (CDIM > 1) s_colv[tid] = make_float4(cw.y, cw.z, cw.w, 0.f);
+            }
+            s_geo2[tid] = make_float4(cc, op, be, cw.x);
+            if constexpr (!kColVec) {
 #pragma unroll
                 for (int k = 0; k < CDIM; ++k) s_col[k][tid] = cp[k];
             }
             float hx, hy;
             support_box(ca, cb, cc, hx, hy);
             const uint32_t sub_mask = g_ok ? subblock_mask_exact<SB>(xy.x, xy.y, ca, cb, cc, hx, hy, x0, y0) : 0u;
-            s_mask[tid] = sub_mask;
+            // how the blend may evaluate the entry: plain (alpha cannot reach the
+            // 0.999 clamp), ordinary (finite values, 0 <= alpha, and no sigma that
+            // underflows to -0: dx is 0 or at least 2^-25), or only by the general
+            // code
+            const bool ordinary =
+                op >= 0.f && op < 1e30f && be >= 0.f && be < 1e30f && ca >= 1e-12f && cc >= 1e-12f;
+            const bool plain = ordinary && op <= kNoClampOpacity;
+            staged_mask = sub_mask | (ordinary ? 0u : kGeneralBit) | (plain ? 0u : kClampBit);
             if (entry_masks && write_meta) {  // for the backward
                 typedef typename EntryMask<SB>::type EM;
                 static_cast<EM *>(entry_masks)[batch_start + tid] = (EM)sub_mask;
             }
         }
+        s_mask[tid] = staged_mask;
         __syncthreads();
         // ---- per-wave compaction of the batch to this sub-block's primitives
         // (a list in LDS measured faster here than walking ballot bits, whose
         // scalar bookkeeping competes with this short loop body)
         int n_mine = 0;
-        for (int c0 = 0; c0 < cnt; c0 += 64) {
-            const int e = c0 + lane;
-            const bool hit = e < cnt && ((s_mask[e] >> wave) & 1u);
-            const uint64_t bal = __ballot(hit);
-            if (hit) {
-                const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-                s_list[wave][n_mine + __popcll(bal & lt)] = (uint32_t)(e * 16);
+        uint64_t general = 0ull, clamp = 0ull;  // any such entry among them
+        constexpr int CH = NW < 4 ? NW : 4;     // chunks of 64 whose masks are read together
+        for (int c0 = 0; c0 < cnt; c0 += 64 * CH) {
+            uint32_t m[CH];
+#pragma unroll
+            for (int u = 0; u < CH; ++u) m[u] = s_mask[c0 + 64 * u + lane];
+#pragma unroll
+            for (int u = 0; u < CH; ++u) {
+                const bool hit = (m[u] >> wave) & 1u;
+                const uint64_t bal = __ballot(hit);
+                general |= __ballot(hit && (m[u] & kGeneralBit));
+                clamp |= __ballot(hit && (m[u] & kClampBit));
+                if (hit)
+                    s_list[wave][n_mine + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
+                                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] =
+                        (uint32_t)((c0 + 64 * u + lane) * 16);
+                n_mine += __popcll(bal);
             }
-            n_mine += __popcll(bal);
         }
         // (s_list[wave] is written and read by this wave only: LDS is in order)
         // ---- front-to-back blend over the compacted list, branch-free per
-        // pixel: lanes that skip the primitive blend alpha = 0.  The loop body
-        // has no branch at all (the all-done exit is checked once per 8
-        // primitives): skipping the body when no lane hits the primitive cost
-        // more in scalar mask bookkeeping than it saved (1.39 vs 1.18 ms at
-        // 1080p / 1M primitives)
+        // pixel: lanes that skip the primitive blend alpha = 0 (skipping the body
+        // when no lane hits the primitive cost more in scalar mask bookkeeping
+        // than it saved: 1.39 vs 1.18 ms at 1080p / 1M primitives)
         int cur_off = -1;  // byte offset of this batch's last contributor
+        auto rec_at = [&](const int off, float4 &g1, float4 &g2, float4 &cv) {
+            g1 = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(s_geo) + off);
+            g2 = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(s_geo2) + off);
+            cv = make_float4(g2.w, 0.f, 0.f, 0.f);
+            if constexpr (kColVec && CDIM > 1) {
+                const char *rest = reinterpret_cast<const char *>(s_colv) + off;
+                if constexpr (CDIM == 2) {
+                    cv.y = *reinterpret_cast<const float *>(rest);
+                } else if constexpr (CDIM == 3) {
+                    const float2 c2 = *reinterpret_cast<const float2 *>(rest);
+                    cv.y = c2.x; cv.z = c2.y;
+                } else {
+                    const float4 c4 = *reinterpret_cast<const float4 *>(rest);
+                    cv.y = c4.x; cv.z = c4.y; cv.w = c4.z;
+                }
+            }
+        };
+        // Lists without an entry for the general code, K primitives at a time.
+        // A pixel's end is rare: it is looked for once per step (T only falls, so
+        // the last T of the step tells), and the step is redone with it if any
+        // lane has one.  Otherwise a lane that a primitive misses blends
+        // alpha = 0 with no further selects; a pixel that is done misses all.
+        // The two quarter-rate instructions issue at raised priority: between
+        // them other waves' plain FP32 instructions go out in pairs, which a
+        // transcendental of another wave in their middle prevents (2.65 against
+        // 4.05 cycles per instruction for this mix).  One primitive at a time
+        // with all selects (the general code) took 978 us at 1080p / 1M, this 880.
+        auto ordinary_list = [&](auto clamp_tag) {
+            constexpr bool CLAMP = decltype(clamp_tag)::value;
+            constexpr int K = UBS_FWD_STEP;
+            for (int k0 = 0; k0 < n_mine; k0 += K) {
+                int off[K];
+                float4 g1[K], g2[K], cv[K];
+#pragma unroll
+                for (int u = 0; u < K; u += 2) {
+                    const uint2 both = *reinterpret_cast<const uint2 *>(&s_list[wave][k0 + u]);
+                    off[u] = (int)both.x;
+                    off[u + 1] = (int)both.y;
+                }
+#pragma unroll
+                for (int u = 0; u < K; ++u) rec_at(off[u], g1[u], g2[u], cv[u]);
+                bool ok[K];
+                float lg[K], alpha[K], Tn[K + 1];
+#pragma unroll
+                for (int u = 0; u < K; ++u) {
+                    const float dx = g1[u].x - bx, dy = g1[u].y - py;
+                    const float sigma =
+                        __builtin_fmaf(g1[u].w * dx, dy, __builtin_fmaf(g1[u].z * dx, dx, (g2[u].x * dy) * dy));
+                    ok[u] = __float_as_uint(sigma) < 0x3f800000u;  // 0 <= sigma < 1 (sigma is not -0 here)
+                    lg[u] = 1.f - sigma;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+                for (int u = 0; u < K; ++u) lg[u] = __builtin_amdgcn_logf(lg[u]);
+#pragma unroll
+                for (int u = 0; u < K; ++u) lg[u] = __builtin_amdgcn_exp2f(g2[u].z * lg[u]);
+                __builtin_amdgcn_s_setprio(0);
+                __builtin_amdgcn_sched_barrier(0);
+                Tn[0] = T;
+                int cur_new = cur_off;
+#pragma unroll
+                for (int u = 0; u < K; ++u) {
+                    const float a0 = g2[u].y * lg[u];
+                    alpha[u] = ok[u] ? (CLAMP ? fminf(0.999f, a0) : a0) : 0.f;
+                    Tn[u + 1] = Tn[u] * (1.f - alpha[u]);
+                    cur_new = ok[u] ? off[u] : cur_new;
+                }
+                if constexpr (STATS) {
+#pragma unroll
+                    for (int u = 0; u < K; ++u) {
+                        st_steps += (uint32_t)(k0 + u < n_mine);
+                        st_live += (uint32_t)(k0 + u < n_mine && bx == bx);
+                        st_sup += (uint32_t)ok[u];
+                        st_take += (uint32_t)ok[u];
+                    }
+                }
+                bool all_done = false;
+                if (__ballot(Tn[K] <= 1e-4f) != 0ull) {
+                    cur_new = cur_off;
+                    float nan_or_x = bx;
+#pragma unroll
+                    for (int u = 0; u < K; ++u) {
+                        // the primitive that would end the pixel is excluded, and all after
+                        // it (alpha = 0 leaves T, which is above the limit)
+                        const bool stop = Tn[u] * (1.f - alpha[u]) <= 1e-4f;
+                        nan_or_x = stop ? __builtin_nanf("") : nan_or_x;
+                        const bool take = ok[u] && nan_or_x == nan_or_x;
+                        if constexpr (STATS) st_take -= (uint32_t)(ok[u] && !take);
+                        alpha[u] = take ? alpha[u] : 0.f;
+                        Tn[u + 1] = Tn[u] * (1.f - alpha[u]);
+                        cur_new = take ? off[u] : cur_new;
+                    }
+                    bx = nan_or_x;
+                    all_done = __ballot(bx == bx) == 0ull;
+                }
+                cur_off = cur_new;
+#pragma unroll
+                for (int u = 0; u < K; ++u) {
+                    const float vis = alpha[u] * Tn[u];
+                    if constexpr (kColVec) {
+                        const float c4[4] = {cv[u].x, cv[u].y, cv[u].z, cv[u].w};
+#pragma unroll
+                        for (int q = 0; q < CDIM; ++q) acc[q] = __builtin_fmaf(c4[q], vis, acc[q]);
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < CDIM; ++q) acc[q] = __builtin_fmaf(s_col[q][off[u] >> 4], vis, acc[q]);
+                    }
+                }
+                T = Tn[K];
+                if (all_done) break;
+            }
+        };
+        if (general == 0ull) {
+            // the list's end up to a whole step: entries that contribute nowhere
+            if (lane < UBS_FWD_STEP && n_mine + lane < ((n_mine + UBS_FWD_STEP - 1) & ~(UBS_FWD_STEP - 1)))
+                s_list[wave][n_mine + lane] = (uint32_t)(BS * 16);
+            if (clamp == 0ull)
+                ordinary_list(std::false_type{});
+            else
+                ordinary_list(std::true_type{});
+            n_mine = 0;  // (nothing left for the general code)
+        }
+        bool done = bx != bx;
         for (int k0 = 0; k0 < n_mine; k0 += 8) {
             if (__ballot(!done) == 0ull) break;  // whole wave done (checked every 8)
             const int kend = min(k0 + 8, n_mine);
@@ -211,40 +379,14 @@ __global__ __launch_bounds__(TS *TS) void raster_fwd_kernel(
                 cur_off = take ? off : cur_off;
                 T = take ? nT : T;
             };
-            auto rec_at = [&](const int off, float4 &g1, float4 &g2, float4 &cv) {
-                g1 = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(s_geo) + off);
-                g2 = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(s_geo2) + off);
-                cv = kColVec ? *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(s_colv) + off)
-                             : make_float4(0.f, 0.f, 0.f, 0.f);
-            };
-#if UBS_FWD_PAIRED_READS
-            // two list entries per LDS read and both records read before either
-            // is blended: half the list reads, one LDS round trip per two steps
-            int k = k0;
-            for (; k + 1 < kend; k += 2) {
-                const uint2 both = *reinterpret_cast<const uint2 *>(&s_list[wave][k]);  // k is even
-                const int off0 = (int)both.x, off1 = (int)both.y;
-                float4 a1, a2, ac, b1, b2, bc;
-                rec_at(off0, a1, a2, ac);
-                rec_at(off1, b1, b2, bc);
-                blend_one(off0, a1, a2, ac);
-                blend_one(off1, b1, b2, bc);
-            }
-            if (k < kend) {
-                const int off = s_list[wave][k];
-                float4 g1, g2, cv;
-                rec_at(off, g1, g2, cv);
-                blend_one(off, g1, g2, cv);
-            }
-#else
             for (int k = k0; k < kend; ++k) {
                 const int off = s_list[wave][k];
                 float4 g1, g2, cv;
                 rec_at(off, g1, g2, cv);
                 blend_one(off, g1, g2, cv);
             }
-#endif
         }
+        bx = done ? __builtin_nanf("") : bx;
         if (cur_off >= 0) cur = batch_start + (cur_off >> 4);
         // T after this batch, for a backward that restarts each batch from it
         if (T_ckpt && write_meta) T_ckpt[ckpt_slot(range_start, logical, b, BS) * BS + tid] = T;
