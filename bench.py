@@ -112,8 +112,7 @@ def algorithmic_bytes(name: str, c: dict, n_isect: int, C: int = 1) -> float:
         tile_passes = math.ceil((end_bit - 32) / 8)
         mode = c.get("sort_mode", "onesweep")
         if name == "ubs_radix_sort_pairs" and mode == "depth_first":
-            # two calls per step: the C*N depth keys (4 passes), the entries on the camera/tile bits
-            return (C * N * (8.0 + 24.0 * 4) + n_isect * (8.0 + 24.0 * tile_passes)) / 2
+            return C * N * (8.0 + 24.0 * 4)  # the C*N depth keys (4 passes)
         if name == "ubs_radix_sort_pairs" and mode == "segmented":
             return n_isect * (8.0 + 24.0 * tile_passes)
         passes = math.ceil(end_bit / 8)
@@ -128,6 +127,10 @@ def algorithmic_bytes(name: str, c: dict, n_isect: int, C: int = 1) -> float:
         return 24.0 * C * N + 12.0 * n_isect
     if name == "ubs_isect_tiles_emit_ordered":  # + the order and prefix reads
         return 36.0 * C * N + 12.0 * n_isect
+    if name == "ubs_isect_bins_plan":  # order and pair record in, record in depth order out
+        return 36.0 * C * N + 4.0 * C * tiles
+    if name == "ubs_isect_bins_place":
+        return 16.0 * C * N + 12.0 * n_isect
     if name == "ubs_isect_depth_keys":
         return 20.0 * C * N
     if name == "ubs_isect_scan_ordered":

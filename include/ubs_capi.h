@@ -332,6 +332,29 @@ int ubs_isect_tiles_emit_ordered_rec(uint32_t C, uint32_t N, const void *pair_re
                                      uint32_t tile_height, int64_t *isect_ids, int32_t *flatten_ids,
                                      int64_t cap, void *stream);
 
+/* The sorted intersection list by direct placement (no sort of the entries):
+ * the pairs in depth order, counted per tile and segment of that order, then
+ * every entry stored at its final place.  Same ids and values as
+ * ubs_isect_tiles_emit_ordered_rec followed by a stable sort on the camera/tile
+ * bits, for visible depths without the sign bit (a negative depth's
+ * sign-extended bits cover the id's upper half).
+ *   ubs_isect_bins_workspace_bytes: 0 where the grid is past the method's
+ *     limits (more than 65535 tile columns or camera rows, or 256 patches of
+ *     32 x 32 tiles);
+ *   ubs_isect_bins_plan: pair_records from ubs_isect_tiles_count_info, order =
+ *     the flat ids sorted by depth; writes the workspace and tile_offsets int32
+ *     [C, th, tw] (as ubs_isect_offset_encode of the list);
+ *   ubs_isect_bins_place: isect_ids and flatten_ids [n_isects]; the same
+ *     workspace and offsets.  Entries past n_isects are not stored.
+ * No counterpart in the reference (it sorts all entries, isect_tiles.cu:224-278). */
+size_t ubs_isect_bins_workspace_bytes(uint32_t C, uint32_t N, uint32_t tile_width, uint32_t tile_height);
+int ubs_isect_bins_plan(uint32_t C, uint32_t N, const void *pair_records, const int32_t *order,
+                        uint32_t tile_size, uint32_t tile_width, uint32_t tile_height, int32_t *tile_offsets,
+                        void *workspace, size_t workspace_bytes, void *stream);
+int ubs_isect_bins_place(uint32_t C, uint32_t N, uint32_t tile_width, uint32_t tile_height,
+                         const int32_t *tile_offsets, const void *workspace, size_t workspace_bytes,
+                         int64_t *isect_ids, int32_t *flatten_ids, int64_t n_isects, void *stream);
+
 /* Bits the (cam, tile) prefix of an isect id occupies: 32 + this = end_bit. */
 uint32_t ubs_isect_prefix_bits(uint32_t C, uint32_t tile_width, uint32_t tile_height);
 

@@ -279,8 +279,10 @@ def set_isect_sort_mode(mode: str) -> None:
     """How isect ids reach their sorted order; every mode gives the same
     ids and values, bit for bit:
       depth_first (default): the (camera, primitive) pairs sorted by depth
-        once, entries emitted in that order, then two onesweep passes over
-        the camera/tile bits;
+        once, then every entry stored at its place in the list (tile by tile,
+        in that order); with a negative visible depth, or a tile grid past
+        that method's limits, entries emitted in that order, then two
+        onesweep passes over the camera/tile bits;
       segmented: entries in primitive order, onesweep over the camera/tile
         bits, then a per-tile depth sort in LDS;
       onesweep: onesweep passes over every byte of the ids."""
@@ -348,7 +350,7 @@ def isect_read_info(states) -> list:
 class IsectState:
     """The intersection stage up to the host read of n_isects (see isect_begin)."""
     __slots__ = ("means2d", "radii", "depths", "tile_size", "tile_width", "tile_height", "sort", "tpg", "cum",
-                 "info", "info_host", "ready", "order", "prec", "C", "N")
+                 "info", "info_host", "ready", "order", "prec", "bins", "offsets", "C", "N")
 
 
 def isect_begin(means2d: Tensor, radii: Tensor, depths: Tensor, tile_size: int, tile_width: int, tile_height: int,
@@ -392,19 +394,21 @@ def isect_begin(means2d: Tensor, radii: Tensor, depths: Tensor, tile_size: int, 
     _call("ubs_isect_tiles_count_info", C, N, ptr(means2d), ptr(radii), ptr(depths), tile_size, tile_width,
           tile_height, ptr(S.tpg), ptr(S.cum), ptr(S.info), ptr(_late_status(dev)), ptr(dkeys), ptr(dvals),
           ptr(S.prec), ptr(ws), ws_bytes, st)
-    S.order = S.info_host = S.ready = None
+    S.order = S.info_host = S.ready = S.bins = S.offsets = None
     if depth_first:
-        # the info leaves for the host first; the depth sort and its scan
-        # run during the round trip
+        # the info leaves for the host first; the depth sort and what follows
+        # from it run during the round trip
         S.info_host = torch.empty((3,), dtype=torch.int64, pin_memory=True)
         S.info_host.copy_(S.info, non_blocking=True)
         S.ready = torch.cuda.Event()
         S.ready.record(torch.cuda.current_stream(dev))
         _, S.order = radix_sort_pairs(dkeys, dvals, 0, 32, status_out=_late_status(dev))
-        S.cum = torch.empty((C * N,), dtype=torch.int64, device=dev)
-        ows = int(L.ubs_isect_ordered_workspace_bytes(C, N))
-        ow = torch.empty((ows,), dtype=torch.uint8, device=dev)
-        _call("ubs_isect_scan_ordered", C, N, ptr(S.tpg), ptr(S.order), ptr(S.cum), ptr(ow), ows, st)
+        bins_bytes = int(L.ubs_isect_bins_workspace_bytes(C, N, tile_width, tile_height))
+        if bins_bytes:
+            S.bins = torch.empty((bins_bytes,), dtype=torch.uint8, device=dev)
+            S.offsets = torch.empty((C, tile_height, tile_width), dtype=torch.int32, device=dev)
+            _call("ubs_isect_bins_plan", C, N, ptr(S.prec), ptr(S.order), tile_size, tile_width, tile_height,
+                  ptr(S.offsets), ptr(S.bins), bins_bytes, st)
     return S
 
 
@@ -416,9 +420,18 @@ def isect_finish(S: IsectState, n_isects: int, packed: int):
     tw, th, ts = S.tile_width, S.tile_height, S.tile_size
     isect_ids = torch.empty((n_isects,), dtype=torch.int64, device=dev)
     flatten_ids = torch.empty((n_isects,), dtype=torch.int32, device=dev)
-    if n_isects and S.order is not None:
+    if S.bins is not None and packed >= 0:  # (a negative depth's bits cover the tile in the ids: sorted below)
         # capped at n_isects: the depth order may come from a sort whose
         # status the host has not read yet
+        _call("ubs_isect_bins_place", C, S.N, tw, th, ptr(S.offsets), ptr(S.bins), S.bins.numel(), ptr(isect_ids),
+              ptr(flatten_ids), n_isects, st)
+        return S.tpg, isect_ids, flatten_ids, S.offsets
+    if n_isects and S.order is not None:
+        S.cum = torch.empty((C * S.N,), dtype=torch.int64, device=dev)
+        ows = int(L.ubs_isect_ordered_workspace_bytes(C, S.N))
+        ow = torch.empty((ows,), dtype=torch.uint8, device=dev)
+        _call("ubs_isect_scan_ordered", C, S.N, ptr(S.tpg), ptr(S.order), ptr(S.cum), ptr(ow), ows, st)
+        # (capped like the placement)
         _call("ubs_isect_tiles_emit_ordered_rec", C, S.N, ptr(S.prec), ptr(S.order), ptr(S.cum), ts, tw, th,
               ptr(isect_ids), ptr(flatten_ids), n_isects, st)
     elif n_isects:
