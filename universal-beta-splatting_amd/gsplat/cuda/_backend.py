@@ -184,19 +184,22 @@ def lib() -> _Lib:
 
 
 def ptr(t: Optional[torch.Tensor]):
-    """Raw device pointer of a contiguous CUDA (HIP) tensor, or None."""
+    """Raw device pointer of a contiguous CUDA (HIP) tensor, or None: a plain
+    int, which the entry points' argtypes convert (a c_void_p object built here
+    first costs 0.2 us a pointer, and a blend passes 45)."""
     if t is None:
         return None
     if not t.is_cuda:
         raise RuntimeError("tensor must be a CUDA (HIP) tensor")
     if not t.is_contiguous():
         raise RuntimeError("tensor must be contiguous")
-    return _vp(t.data_ptr())
+    return t.data_ptr()
 
 
 def stream_of(t: torch.Tensor):
-    """Current HIP stream on the tensor's device."""
-    return _vp(torch.cuda.current_stream(t.device).cuda_stream)
+    """Current HIP stream on the tensor's device, as the raw handle (building
+    torch.cuda's Stream object for it costs 3 us a call)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 _F32, _I32, _I64 = torch.float32, torch.int32, torch.int64
