@@ -10,7 +10,8 @@
 // loss averages S over every pixel and channel.
 //
 // Images are [B, H, W, C] float32 (the rasteriser's layout; no permute).
-// One workgroup per 16x16 pixel tile and (image, channel): the 26x26 input
+// Pixels of up to four channels take the streaming kernels below; wider ones one
+// workgroup per 16x16 pixel tile and (image, channel): the 26x26 input
 // halo is staged in LDS and the window is applied separably (rows, then
 // columns).  The forward writes, per element, dL/dmu1, dL/ds11 and dL/ds12
 // (the derivatives of the averaged SSIM term w.r.t. the three filtered maps
@@ -41,12 +42,45 @@ struct LossLayout {
     int64_t blocks;
 };
 
+// The strips of the streaming kernels: 256 of a row's W C values wide, and
+// chunks x 11 input rows (10 fewer output rows) high.
+constexpr int kStripCols = 256;
+constexpr int kStripBlocks = 700;
+
+struct StripShape {
+    int64_t cols, strips;  // column blocks, strips of an image
+    int chunks;
+    int64_t rows() const { return (int64_t)chunks * kWin - 2 * kHalo; }
+    int64_t blocks() const { return cols * strips; }
+};
+
+// Longer strips repeat less of their halo (4 chunks: 44 input rows for 34 output
+// rows, 2: 22 for 12), shorter ones fill the chip: the longest that leave nearly
+// three workgroups for each of 256 CUs (1080p, three channels: 4 chunks, 736
+// workgroups, forward and backward 66 + 54 us; 6 chunks, 460: 64 + 58; 5, 552:
+// 81 + 64).
+static StripShape strip_shape(int64_t B, int64_t H, int64_t W, int64_t C) {
+    StripShape s{};
+    s.cols = (W * C + kStripCols - 1) / kStripCols;
+    for (s.chunks = 8;; --s.chunks) {
+        s.strips = (H + s.rows() - 1) / s.rows();
+        if (s.chunks == 2 || s.blocks() * B >= kStripBlocks) return s;
+    }
+}
+
+// Pixels of up to four channels stream; wider ones (whose halo of 10 C values
+// would not fit) take the tiles.
+static bool streams(int64_t B, int64_t H, int64_t W, int64_t C) {
+    return C <= 4 && W * C < (1ll << 31) - 4096 && strip_shape(B, H, W, C).blocks() < (1ll << 31) && B < 65536;
+}
+
 static LossLayout loss_layout(int64_t B, int64_t H, int64_t W, int64_t C) {
     LossLayout L{};
     const int64_t tx = (W + kLossTile - 1) / kLossTile, ty = (H + kLossTile - 1) / kLossTile;
-    L.blocks = std::max<int64_t>(tx * ty * B * C, 1);
+    L.blocks = std::max<int64_t>(streams(B, H, W, C) ? strip_shape(B, H, W, C).blocks() * B : tx * ty * B * C, 1);
     L.partial_off = 0;
-    size_t off = (size_t)std::max<int64_t>(L.blocks, 1024) * 2 * sizeof(float);  // also the L1 pass's 1024 blocks
+    // also the L1 pass's 1024 blocks, and the tiles of a misaligned one
+    size_t off = (size_t)std::max<int64_t>(std::max<int64_t>(L.blocks, tx * ty * B * C), 1024) * 2 * sizeof(float);
     off = (off + 255) & ~(size_t)255;
     L.dmaps_off = off;
     off += (size_t)3 * B * H * W * C * sizeof(float);
@@ -176,6 +210,223 @@ __global__ __launch_bounds__(256) void loss_fwd_kernel(int64_t B, int64_t H, int
         const int64_t blk = bc * gridDim.x + blockIdx.x;
         partial[2 * blk] = s_sum;
         partial[2 * blk + 1] = l1_sum;
+    }
+}
+
+// The streaming kernels (pixels of up to four channels).  A row of the image is
+// W C consecutive values and the window's taps along it are C values apart, so a
+// thread takes one of 256 consecutive values (coalesced, whatever the channel)
+// and walks down the rows: 11 input rows at a time are staged in LDS with a halo
+// of 5 C values on either side, a row is filtered along itself from there, and
+// the last 11 filtered rows stay in registers for the filter across rows (the
+// loop over 11 rows is unrolled, so a row's place in the ring is a constant).
+// Bound by VALU issue and its dependent chains at 2-3 waves per SIMD (the ring and
+// the chunk under way take 170-210 registers): about 160 instructions an element
+// in the forward, 1.3 times for the halo rows.  Forward and backward at 1080p,
+// three channels: 66 and 54 us, where tiles of 16 x 16 pixels of one channel, which
+// read 2.6 times their pixels at a stride of C values and pass every filtered row
+// through LDS, took 124 and 111.  (Held to 128 registers: 88 and 75.)
+//
+// 11 rows of M images: a thread holds its own column's values and its share of the
+// two halos' (11 x 10 C values an image).  A row's address is the same for the
+// whole workgroup, so that a load needs only the column's 32-bit offset.
+template <int C, int M>
+struct Chunk {
+    static constexpr int kPad = kHalo * C, kRow = kStripCols + 2 * kPad;
+    static constexpr int kHaloAll = M * kWin * 2 * kPad, kPer = (kHaloAll + kStripCols - 1) / kStripCols;
+    float own[M][kWin], halo[kPer];
+
+    __device__ __forceinline__ void load(const float *const (&img)[M], int64_t first, int64_t H, int64_t len,
+                                         int64_t f0) {
+        const int tid = threadIdx.x;
+        const bool col = f0 + tid < len;
+        const uint32_t off = (uint32_t)(col ? f0 + tid : 0) * 4u;
+#pragma unroll
+        for (int r = 0; r < kWin; ++r) {
+            const int64_t i = first + r;
+            const bool row = i >= 0 && i < H;  // zero padding
+            const int64_t at = (row ? i : 0) * len;
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const float v = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(img[m] + at) + off);
+                own[m][r] = row && col ? v : 0.f;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            const int k = tid + u * kStripCols, m = k / (kWin * 2 * kPad), q = k % (2 * kPad);
+            const int64_t i = first + k / (2 * kPad) % kWin, f = q < kPad ? f0 - kPad + q : f0 + kStripCols + q - kPad;
+            const bool ok = k < kHaloAll && i >= 0 && i < H && f >= 0 && f < len;
+            const float *const src = m == 0 ? img[0] : m == 1 || M == 2 ? img[M > 1 ? 1 : 0] : img[M - 1];
+            halo[u] = ok ? src[i * len + f] : 0.f;
+        }
+    }
+    __device__ __forceinline__ void store(float (&s)[M][kWin][kRow]) const {
+        const int tid = threadIdx.x;
+#pragma unroll
+        for (int r = 0; r < kWin; ++r)
+#pragma unroll
+            for (int m = 0; m < M; ++m) s[m][r][kPad + tid] = own[m][r];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            const int k = tid + u * kStripCols, q = k % (2 * kPad);
+            if (k < kHaloAll) s[k / (kWin * 2 * kPad)][k / (2 * kPad) % kWin][q < kPad ? q : q + kStripCols] = halo[u];
+        }
+    }
+};
+
+template <int C>
+__global__ __launch_bounds__(kStripCols, 2) void ssim_fwd_kernel(int64_t H, int64_t len, int64_t cols, int chunks,
+                                                              const float *__restrict__ x,
+                                                              const float *__restrict__ y, GaussWin win, float k,
+                                                              int64_t n_el, float *__restrict__ partial,
+                                                              float *__restrict__ dmaps) {
+    __shared__ float sxy[2][kWin][Chunk<C, 2>::kRow];
+    __shared__ double red[2][kStripCols / 64];
+    const int tid = threadIdx.x;
+    const int64_t strip = blockIdx.x / cols, f0 = (int64_t)(blockIdx.x % cols) * kStripCols, f = f0 + tid;
+    const uint32_t f32 = (uint32_t)f;
+    const int64_t rows = (int64_t)chunks * kWin - 2 * kHalo, i0 = strip * rows;
+    const int64_t img = (int64_t)blockIdx.y * H * len;
+    x += img;
+    y += img;
+    dmaps += img;
+    float h0[kWin], h1[kWin], h2[kWin], h3[kWin], h4[kWin];  // the last 11 filtered rows
+    const float *const both[2] = {x, y};
+    Chunk<C, 2> next;  // (loaded while the chunk before it is filtered)
+    next.load(both, i0 - kHalo, H, len, f0);
+    double s_sum = 0.0, l1_sum = 0.0;
+    for (int ch = 0; ch < chunks; ++ch) {
+        __syncthreads();
+        next.store(sxy);
+        __syncthreads();
+        const int64_t ir = i0 - kHalo + (int64_t)ch * kWin;  // image row of the chunk's first
+        if (ch + 1 < chunks) next.load(both, ir + kWin, H, len, f0);
+        float s_part = 0.f, l1_part = 0.f;
+#pragma unroll
+        for (int r = 0; r < kWin; ++r) {
+            __builtin_amdgcn_sched_barrier(0);
+            float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f, a4 = 0.f;
+#pragma unroll
+            for (int t = 0; t < kWin; ++t) {
+                const float g = win.g[t], u = sxy[0][r][tid + t * C], v = sxy[1][r][tid + t * C];
+                const float gu = g * u, gv = g * v;
+                a0 += gu;
+                a1 += gv;
+                a2 = __builtin_fmaf(gu, u, a2);
+                a3 = __builtin_fmaf(gv, v, a3);
+                a4 = __builtin_fmaf(gu, v, a4);
+                if (t == kHalo && ir + r >= i0 && ir + r < i0 + rows) l1_part += fabsf(u - v);  // (0 outside the image)
+            }
+            h0[r] = a0;
+            h1[r] = a1;
+            h2[r] = a2;
+            h3[r] = a3;
+            h4[r] = a4;
+            if (ch == 0 && r < kWin - 1) continue;  // the first output row needs 11
+            float m1 = 0.f, m2 = 0.f, e11 = 0.f, e22 = 0.f, e12 = 0.f;
+#pragma unroll
+            for (int t = 0; t < kWin; ++t) {
+                constexpr int n = kWin;
+                const float g = win.g[t];
+                const int q = (r + 1 + t) % n;  // oldest first
+                m1 = __builtin_fmaf(g, h0[q], m1);
+                m2 = __builtin_fmaf(g, h1[q], m2);
+                e11 = __builtin_fmaf(g, h2[q], e11);
+                e22 = __builtin_fmaf(g, h3[q], e22);
+                e12 = __builtin_fmaf(g, h4[q], e12);
+            }
+            const int64_t i = ir + r - kHalo;  // the output row
+            if (i < H && f < len) {
+                const float mu11 = m1 * m1, mu22 = m2 * m2, mu12 = m1 * m2;
+                const float s11 = e11 - mu11, s22 = e22 - mu22, s12 = e12 - mu12;
+                const float A1 = 2.f * mu12 + kC1, A2 = 2.f * s12 + kC2;
+                const float B1 = mu11 + mu22 + kC1, B2 = s11 + s22 + kC2;
+                const float D = B1 * B2;
+                const float Sv = (A1 * A2) / D;
+                s_part += Sv;
+                // derivatives of S w.r.t. mu1, E[x^2] and E[xy] (loss_utils.py:56-80)
+                const float dmu1 = (2.f * m2 * (A2 - A1) - 2.f * m1 * Sv * (B2 - B1)) / D;
+                const float ds11 = -Sv / B2;
+                const float ds12 = 2.f * A1 / D;
+                float *const d = dmaps + i * len;
+                d[f32] = k * dmu1;
+                d[n_el + f32] = k * ds11;
+                d[2 * n_el + f32] = k * ds12;
+            }
+        }
+        s_sum += (double)s_part;
+        l1_sum += (double)l1_part;
+    }
+    if (f >= len) l1_sum = 0.0;  // (another strip's halo)
+    for (int o = 32; o > 0; o >>= 1) {
+        s_sum += __shfl_xor(s_sum, o, 64);
+        l1_sum += __shfl_xor(l1_sum, o, 64);
+    }
+    if ((tid & 63) == 0) {
+        red[0][tid >> 6] = s_sum;
+        red[1][tid >> 6] = l1_sum;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        const int64_t blk = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+        partial[2 * blk] = (float)((red[0][0] + red[0][1]) + (red[0][2] + red[0][3]));
+        partial[2 * blk + 1] = (float)((red[1][0] + red[1][1]) + (red[1][2] + red[1][3]));
+    }
+}
+
+template <int C>
+__global__ __launch_bounds__(kStripCols, 3) void ssim_bwd_kernel(int64_t H, int64_t len, int64_t cols, int chunks,
+                                                              const float *__restrict__ x,
+                                                              const float *__restrict__ y, GaussWin win, float l1,
+                                                              int64_t n_el, const float *__restrict__ v_loss,
+                                                              const float *__restrict__ dmaps,
+                                                              float *__restrict__ v_x) {
+    __shared__ float sd[3][kWin][Chunk<C, 3>::kRow];
+    const int tid = threadIdx.x;
+    const int64_t strip = blockIdx.x / cols, f0 = (int64_t)(blockIdx.x % cols) * kStripCols, f = f0 + tid;
+    const uint32_t f32 = (uint32_t)f;
+    const int64_t i0 = strip * ((int64_t)chunks * kWin - 2 * kHalo);
+    const int64_t img = (int64_t)blockIdx.y * H * len;
+    x += img;
+    y += img;
+    v_x += img;
+    dmaps += img;
+    const float vl = v_loss[0];
+    float h[3][kWin];
+    const float *const maps[3] = {dmaps, dmaps + n_el, dmaps + 2 * n_el};
+    Chunk<C, 3> next;
+    next.load(maps, i0 - kHalo, H, len, f0);
+    for (int ch = 0; ch < chunks; ++ch) {
+        __syncthreads();
+        next.store(sd);
+        __syncthreads();
+        const int64_t ir = i0 - kHalo + (int64_t)ch * kWin;
+        if (ch + 1 < chunks) next.load(maps, ir + kWin, H, len, f0);
+#pragma unroll
+        for (int r = 0; r < kWin; ++r) {
+            __builtin_amdgcn_sched_barrier(0);
+            float a[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < kWin; ++t)
+#pragma unroll
+                for (int m = 0; m < 3; ++m) a[m] = __builtin_fmaf(win.g[t], sd[m][r][tid + t * C], a[m]);
+#pragma unroll
+            for (int m = 0; m < 3; ++m) h[m][r] = a[m];
+            if (ch == 0 && r < kWin - 1) continue;
+            float b[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < kWin; ++t)
+#pragma unroll
+                for (int m = 0; m < 3; ++m) b[m] = __builtin_fmaf(win.g[t], h[m][(r + 1 + t) % kWin], b[m]);
+            const int64_t i = ir + r - kHalo;
+            if (i < H && f < len) {
+                const int64_t at = i * len;
+                const float xv = x[at + f32], yv = y[at + f32], d = xv - yv;
+                const float sgn = d > 0.f ? 1.f : (d < 0.f ? -1.f : 0.f);
+                v_x[at + f32] = vl * (l1 * sgn + (b[0] + 2.f * xv * b[1] + yv * b[2]));
+            }
+        }
     }
 }
 
@@ -348,6 +599,21 @@ int ubs_image_loss_fwd(int64_t B, int64_t H, int64_t W, int64_t C, const float *
     }
     const dim3 grid((unsigned)tiles, (unsigned)(B * C));
     const GaussWin win = gauss_window();
+    if (ssim && streams(B, H, W, C)) {
+        const StripShape s = strip_shape(B, H, W, C);
+        const dim3 g((unsigned)s.blocks(), (unsigned)B);
+        const float k = -lambda_dssim * (1.f / (float)n);  // d loss / d S at every element
+#define UBS_SSIM_FWD(K)                                                                                              \
+    case K:                                                                                                          \
+        ssim_fwd_kernel<K><<<g, kStripCols, 0, st>>>(H, W * C, s.cols, s.chunks, img, gt, win, k, n, partial, dmaps); \
+        break;
+        switch (C) { UBS_SSIM_FWD(1) UBS_SSIM_FWD(2) UBS_SSIM_FWD(3) UBS_SSIM_FWD(4) }
+#undef UBS_SSIM_FWD
+        UBS_LAUNCH_CHECK("ssim_fwd_kernel");
+        loss_finish_kernel<<<1, 256, 0, st>>>(L.blocks, partial, lambda_dssim, (double)n, 1, loss);
+        UBS_LAUNCH_CHECK("loss_finish_kernel");
+        return UBS_OK;
+    }
     if (ssim)
         loss_fwd_kernel<true><<<grid, 256, 0, st>>>(B, H, W, C, img, gt, win, lambda_dssim, 1.f / (float)n, partial,
                                                     dmaps);
@@ -355,7 +621,7 @@ int ubs_image_loss_fwd(int64_t B, int64_t H, int64_t W, int64_t C, const float *
         loss_fwd_kernel<false><<<grid, 256, 0, st>>>(B, H, W, C, img, gt, win, lambda_dssim, 1.f / (float)n,
                                                      partial, dmaps);
     UBS_LAUNCH_CHECK("loss_fwd_kernel");
-    loss_finish_kernel<<<1, 256, 0, st>>>(L.blocks, partial, lambda_dssim, (double)n, ssim ? 1 : 0, loss);
+    loss_finish_kernel<<<1, 256, 0, st>>>(tiles * B * C, partial, lambda_dssim, (double)n, ssim ? 1 : 0, loss);
     UBS_LAUNCH_CHECK("loss_finish_kernel");
     return UBS_OK;
 }
@@ -387,6 +653,20 @@ int ubs_image_loss_bwd(int64_t B, int64_t H, int64_t W, int64_t C, const float *
     }
     const dim3 grid((unsigned)tiles, (unsigned)(B * C));
     const GaussWin win = gauss_window();
+    if (lambda_dssim > 0.f && streams(B, H, W, C)) {
+        const StripShape s = strip_shape(B, H, W, C);
+        const dim3 g((unsigned)s.blocks(), (unsigned)B);
+        const float l1 = (1.f - lambda_dssim) * (1.f / (float)n);
+#define UBS_SSIM_BWD(K)                                                                                           \
+    case K:                                                                                                       \
+        ssim_bwd_kernel<K><<<g, kStripCols, 0, st>>>(H, W * C, s.cols, s.chunks, img, gt, win, l1, n, v_loss,     \
+                                                     dmaps, v_img);                                               \
+        break;
+        switch (C) { UBS_SSIM_BWD(1) UBS_SSIM_BWD(2) UBS_SSIM_BWD(3) UBS_SSIM_BWD(4) }
+#undef UBS_SSIM_BWD
+        UBS_LAUNCH_CHECK("ssim_bwd_kernel");
+        return UBS_OK;
+    }
     if (lambda_dssim > 0.f)
         loss_bwd_kernel<true><<<grid, 256, 0, st>>>(B, H, W, C, img, gt, win, lambda_dssim, 1.f / (float)n, v_loss,
                                                     dmaps, v_img);
