@@ -82,7 +82,8 @@ ENTRY_ALIASES = {"ubs_rasterize_to_pixels_bwd_reuse": "ubs_rasterize_to_pixels_b
                  "ubs_isect_tiles_emit_ordered_cap": "ubs_isect_tiles_emit_ordered",
                  "ubs_isect_tiles_emit_ordered_rec": "ubs_isect_tiles_emit_ordered",
                  "ubs_radix_sort_pairs_flag": "ubs_radix_sort_pairs",
-                 "ubs_isect_tiles_count_info": "ubs_isect_tiles_count_range"}
+                 "ubs_isect_tiles_count_info": "ubs_isect_tiles_count_range",
+                 "ubs_isect_tiles_count_depths": "ubs_isect_tiles_count_range"}
 
 
 def launch_durations(timer) -> dict:

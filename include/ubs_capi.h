@@ -323,6 +323,15 @@ int ubs_isect_tiles_count_info(uint32_t C, uint32_t N, const float *means2d, con
                                int32_t *depth_vals, void *pair_records, void *workspace,
                                size_t workspace_bytes, void *stream);
 
+/* ubs_isect_tiles_count_info without the running sum of the counts, for callers
+ * whose entries are placed by ubs_isect_bins_*; depth_keys, depth_vals and
+ * pair_records are required.  No counterpart in the reference. */
+int ubs_isect_tiles_count_depths(uint32_t C, uint32_t N, const float *means2d, const int32_t *radii,
+                                 const float *depths, uint32_t tile_size, uint32_t tile_width,
+                                 uint32_t tile_height, int32_t *tiles_per_gauss, int64_t *info,
+                                 const int64_t *status_in, int64_t *depth_keys, int32_t *depth_vals,
+                                 void *pair_records, void *workspace, size_t workspace_bytes, void *stream);
+
 /* ubs_isect_tiles_emit_ordered_cap reading each pair's centre, radius and
  * depth from the 16-byte pair records ubs_isect_tiles_count_info wrote (one
  * gather per pair in depth order instead of three).  No counterpart in the

@@ -72,6 +72,9 @@ _SIGNATURES = {
     "ubs_isect_tiles_count_info": (
         _c_int, [_c_u32, _c_u32, _vp, _vp, _vp, _c_u32, _c_u32, _c_u32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                  _c_size, _vp]),
+    "ubs_isect_tiles_count_depths": (
+        _c_int, [_c_u32, _c_u32, _vp, _vp, _vp, _c_u32, _c_u32, _c_u32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_size,
+                 _vp]),
     "ubs_isect_tiles_emit_ordered_rec": (
         _c_int, [_c_u32, _c_u32, _vp, _vp, _vp, _c_u32, _c_u32, _c_u32, _vp, _vp, _c_i64, _vp]),
     "ubs_isect_bins_workspace_bytes": (_c_size, [_c_u32, _c_u32, _c_u32, _c_u32]),

@@ -379,7 +379,6 @@ def isect_begin(means2d: Tensor, radii: Tensor, depths: Tensor, tile_size: int, 
     S.means2d, S.radii, S.depths, S.C, S.N = means2d, radii, depths, C, N
     S.tile_size, S.tile_width, S.tile_height, S.sort = tile_size, tile_width, tile_height, sort
     S.tpg = torch.empty((C, N), dtype=torch.int32, device=dev)
-    S.cum = torch.empty((C * N,), dtype=torch.int64, device=dev)
     # [n_isects, (~min depth bits, max depth bits) as two uint32, sort status],
     # written by the count kernels and read in one sync
     S.info = torch.empty((3,), dtype=torch.int64, device=dev)
@@ -391,9 +390,16 @@ def isect_begin(means2d: Tensor, radii: Tensor, depths: Tensor, tile_size: int, 
     dvals = torch.empty((C * N,), dtype=torch.int32, device=dev) if depth_first else None
     # the emission's per-pair reads (centre, radius, depth) in one 16-byte record
     S.prec = torch.empty((C * N, 4), dtype=torch.float32, device=dev) if depth_first else None
-    _call("ubs_isect_tiles_count_info", C, N, ptr(means2d), ptr(radii), ptr(depths), tile_size, tile_width,
-          tile_height, ptr(S.tpg), ptr(S.cum), ptr(S.info), ptr(_late_status(dev)), ptr(dkeys), ptr(dvals),
-          ptr(S.prec), ptr(ws), ws_bytes, st)
+    if depth_first:
+        S.cum = None  # (only the emission that isect_finish falls back to needs it, in depth order)
+        _call("ubs_isect_tiles_count_depths", C, N, ptr(means2d), ptr(radii), ptr(depths), tile_size, tile_width,
+              tile_height, ptr(S.tpg), ptr(S.info), ptr(_late_status(dev)), ptr(dkeys), ptr(dvals), ptr(S.prec),
+              ptr(ws), ws_bytes, st)
+    else:
+        S.cum = torch.empty((C * N,), dtype=torch.int64, device=dev)
+        _call("ubs_isect_tiles_count_info", C, N, ptr(means2d), ptr(radii), ptr(depths), tile_size, tile_width,
+              tile_height, ptr(S.tpg), ptr(S.cum), ptr(S.info), ptr(_late_status(dev)), None, None, None, ptr(ws),
+              ws_bytes, st)
     S.order = S.info_host = S.ready = S.bins = S.offsets = None
     if depth_first:
         # the info leaves for the host first; the depth sort and what follows
