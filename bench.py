@@ -240,7 +240,7 @@ def _probe_lib():
     lib = ctypes.CDLL(path)
     vp, u32, i64, i32 = ctypes.c_void_p, ctypes.c_uint32, ctypes.c_int64, ctypes.c_int
     lib.ubs_probe_valu.argtypes = [i32, i32, i32, vp, vp]
-    lib.ubs_probe_raster_fwd_stats.argtypes = [u32, u32, i64] + [vp] * 5 + [u32] * 4 + [vp] * 8
+    lib.ubs_probe_raster_fwd_stats.argtypes = [u32, u32, i64] + [vp] * 5 + [u32] * 4 + [vp] * 9
     lib.ubs_probe_raster_bwd_stats.argtypes = [u32, u32, i64] + [vp] * 5 + [u32] * 4 + [vp] * 10
     for f in (lib.ubs_probe_valu, lib.ubs_probe_raster_fwd_stats, lib.ubs_probe_raster_bwd_stats):
         f.restype = i32

@@ -355,14 +355,14 @@ class IsectState:
 
 def isect_begin(means2d: Tensor, radii: Tensor, depths: Tensor, tile_size: int, tile_width: int, tile_height: int,
                 sort: bool = True) -> IsectState:
-    """First half of isect_tiles: tile counts, their prefix, n_isects and the
-    depth range into ``state.info`` ([n_isects, packed range] int64, on the
+    """First half of isect_tiles: tile counts, n_isects and the depth range
+    into ``state.info`` ([n_isects, packed range] int64, on the
     device) and, for the depth-first sort, the depth order of the pairs.
     Nothing waits for the host; several states can be read in one sync
     before their isect_finish calls.  With the depth-first sort the info is
     copied to pinned host memory before the depth sort is queued, so the
-    host read waits for the counts only and the depth sort runs while the
-    host queues the emission; that sort's status then joins the status
+    host read waits for the counts only and the depth sort and the plan of
+    the placement run while the host queues the rest; that sort's status then joins the status
     word the next host read reports."""
     C, N, _ = means2d.shape
     assert means2d.shape == (C, N, 2), means2d.size()
@@ -388,7 +388,7 @@ def isect_begin(means2d: Tensor, radii: Tensor, depths: Tensor, tile_size: int, 
     # the depth-first sort's input (depth bits, flat ids), written by the count pass
     dkeys = torch.empty((C * N,), dtype=torch.int64, device=dev) if depth_first else None
     dvals = torch.empty((C * N,), dtype=torch.int32, device=dev) if depth_first else None
-    # the emission's per-pair reads (centre, radius, depth) in one 16-byte record
+    # what the placement (or emission) reads of a pair (centre, radius, depth) in one 16-byte record
     S.prec = torch.empty((C * N, 4), dtype=torch.float32, device=dev) if depth_first else None
     if depth_first:
         S.cum = None  # (only the emission that isect_finish falls back to needs it, in depth order)
