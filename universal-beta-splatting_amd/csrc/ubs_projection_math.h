@@ -223,18 +223,25 @@ __device__ __forceinline__ void proj_bwd_body(const float *__restrict__ means, c
                                               const float *__restrict__ v_comp, float (&vmean)[3],
                                               float (&vS)[3][3], float (&vR)[3][3], float (&vt)[3]) {
     const float P[2][2] = {{cn[0], cn[1]}, {cn[1], cn[2]}};
-    const float vP[2][2] = {{vc[0], vc[1] * 0.5f}, {vc[1] * 0.5f, vc[2]}};
     float vcov2[2][2];
     {
-        float tmp[2][2];
+        // -P vP P in FP64, rounded once.  Of a needle's conic gradient (moments of
+        // offsets of a hundred pixels) the product keeps the part across it, 1e-4
+        // of the entries: in FP32 that part came out with 1e-3 of rounding, another
+        // one for every last bit of the gradient (the blend adds it with atomics),
+        // and a needle's rotation gradient moved by 2e-3 of the gradient's rms
+        // between two runs on the same inputs (now 4e-4 at most).
+        const double Pd[2][2] = {{(double)cn[0], (double)cn[1]}, {(double)cn[1], (double)cn[2]}};
+        const double vP[2][2] = {{(double)vc[0], 0.5 * (double)vc[1]}, {0.5 * (double)vc[1], (double)vc[2]}};
+        double tmp[2][2];
 #pragma unroll
         for (int r = 0; r < 2; ++r)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) tmp[r][s] = P[r][0] * vP[0][s] + P[r][1] * vP[1][s];
+            for (int s = 0; s < 2; ++s) tmp[r][s] = Pd[r][0] * vP[0][s] + Pd[r][1] * vP[1][s];
 #pragma unroll
         for (int r = 0; r < 2; ++r)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) vcov2[r][s] = -(tmp[r][0] * P[0][s] + tmp[r][1] * P[1][s]);
+            for (int s = 0; s < 2; ++s) vcov2[r][s] = (float)-(tmp[r][0] * Pd[0][s] + tmp[r][1] * Pd[1][s]);
     }
     if (v_comp) {
         const float cmpv = *comp, vcp = *v_comp;
