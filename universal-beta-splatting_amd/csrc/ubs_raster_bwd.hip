@@ -232,8 +232,8 @@ __global__ __launch_bounds__(64, UBS_BWD_WAVES_PER_EU) void raster_bwd_kernel(
     const int32_t range_end = min(max(off_hi, range_start), (int32_t)n_isects);
 
     // ---- per-pixel state: thread -> pixel `lane` of the sub-block.  Pixels
-    // outside the image get T = 0 and zero gradients: whatever is evaluated
-    // there adds exact zeros.
+    // outside the image get T = 0, zero gradients and no last contributor: no
+    // primitive is valid there.
     const int32_t bin_final = inside ? last_ids[pix] : 0;
     bool finite = true;  // no infinity or NaN in the incoming gradients
     {
@@ -255,9 +255,12 @@ __global__ __launch_bounds__(64, UBS_BWD_WAVES_PER_EU) void raster_bwd_kernel(
     }
     const bool all_finite = __ballot(finite) == ~0ull;
     // the largest last contributor over the wave bounds the useful range; up
-    // to the smallest, every pixel is still blending
+    // to the smallest, every pixel is still blending.  A pixel outside the image
+    // never is (nothing stopped at T <= 1e-4 there, so the product of 1 / (1 -
+    // alpha) over a stack of opaque primitives would pass FP32's range, and 0 x
+    // inf is NaN): a sub-block over the image's edge takes the general tests.
     const int32_t wave_bin_max = __builtin_amdgcn_readfirstlane(wave_max_i32(bin_final));
-    const int32_t wave_bin_min = -__builtin_amdgcn_readfirstlane(wave_max_i32(inside ? -bin_final : INT32_MIN + 1));
+    const int32_t wave_bin_min = -__builtin_amdgcn_readfirstlane(wave_max_i32(inside ? -bin_final : INT32_MAX));
     // the lane's pixels: x offsets pxb + r, y offset pyb + the step's
     const float pxb = (float)(sx0 + (uint32_t)(R == 4 ? 4 * (row & 1) : 2 * row)) + 0.5f;
     const float pyb = (float)(sy0 + (uint32_t)(R == 4 ? row >> 1 : 0)) + 0.5f;
