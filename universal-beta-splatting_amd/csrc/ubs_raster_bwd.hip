@@ -462,7 +462,8 @@ __global__ __launch_bounds__(64, UBS_BWD_WAVES_PER_EU) void raster_bwd_kernel(
                     T0[r] *= scan[r];  // T before the lane's frontmost primitive
                     Tc[M - 1][r] = (float)T0[r];
                     // (the one behind it: T before it, times 1 - alpha of the front one)
-                    if constexpr (M == 2) Tc[0][r] = Tc[1][r] * oma[1][r];
+                    if constexpr (M == 2)
+                        Tc[0][r] = F64T ? (float)(T0[r] * (TT)(1.0 - (double)alpha[1][r])) : Tc[1][r] * oma[1][r];
 #pragma unroll
                     for (int m = 0; m < M; ++m) {
                         fac[m][r] = alpha[m][r] * Tc[m][r];
