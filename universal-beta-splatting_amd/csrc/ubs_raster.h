@@ -411,6 +411,18 @@ static __global__ void raster_unpack_grads_kernel(uint64_t CN, const float4 *__r
     }
 }
 
+// Positions in a tile's list [start, end), which may end at 2^31 - 1: whether
+// the entry `ahead` places after `at` (start <= at <= end) is in the list, the
+// list's number of batches, and the last entry of the batch that begins at lo <=
+// last.  No sum passes int32.
+__host__ __device__ inline bool list_has(int32_t at, int32_t ahead, int32_t end) { return ahead < end - at; }
+__host__ __device__ inline int32_t list_batches(int32_t start, int32_t end, int32_t batch) {
+    return end > start ? (end - start - 1) / batch + 1 : 0;
+}
+__host__ __device__ inline int32_t list_batch_last(int32_t lo, int32_t last, int32_t batch) {
+    return last - lo < batch - 1 ? last : lo + (batch - 1);
+}
+
 // Transmittance checkpoints (optional): the forward stores every pixel's T
 // after each batch of BS = TS^2 entries of its tile's list, the backward
 // starts each batch from that value instead of carrying the division

@@ -615,7 +615,7 @@ __global__ __launch_bounds__(64, UBS_BWD_WAVES_PER_EU) void raster_bwd_kernel(
     const int32_t nspan = last < range_start ? 0 : T_ckpt ? (last - range_start) / BS + 1 : 1;
     for (int32_t sp = nspan - 1; sp >= 0; --sp) {
         const int32_t lo = range_start + (T_ckpt ? sp * BS : 0);
-        const int32_t hi = T_ckpt ? min(last, lo + BS - 1) : last;
+        const int32_t hi = T_ckpt ? list_batch_last(lo, last, BS) : last;
         if (T_ckpt) {
             if (inside && bin_final >= lo)
                 px.T[lane] = (TT)T_ckpt[ckpt_slot(range_start, logical, sp, BS) * BS +

@@ -129,8 +129,8 @@ __global__ __launch_bounds__(TS *TS) void raster_fwd_kernel(
     for (int k = 0; k < CDIM; ++k) acc[k] = 0.f;
 
     uint32_t st_steps = 0, st_live = 0, st_sup = 0, st_take = 0, st_staged = 0;
-    int32_t g_next = range_start + tid < range_end ? flatten_ids[range_start + tid] : 0;  // of the next batch
-    const int32_t nb = range_end > range_start ? (range_end - range_start + BS - 1) / BS : 0;
+    int32_t g_next = list_has(range_start, tid, range_end) ? flatten_ids[range_start + tid] : 0;  // of the next batch
+    const int32_t nb = list_batches(range_start, range_end, BS);
     for (int32_t b = 0; b < nb; ++b) {
         if (__syncthreads_count(bx != bx) >= BS) break;
         const int32_t batch_start = range_start + b * BS;
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(TS *TS) void raster_fwd_kernel(
         // ---- stage one primitive per thread (its id was loaded a batch ahead: the
         // record's address does not wait for it)
         const int32_t g_raw = g_next;
-        if (batch_start + BS + tid < range_end) g_next = flatten_ids[batch_start + BS + tid];
+        if (list_has(batch_start, BS + tid, range_end)) g_next = flatten_ids[batch_start + BS + tid];
         uint32_t staged_mask = 0;
         if (tid < cnt) {
             // an id outside [0, C N) (only from a sort that gave up) stages
