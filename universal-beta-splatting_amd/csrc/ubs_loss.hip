@@ -37,6 +37,9 @@ constexpr int kSpan = kLossTile + 2 * kHalo;    // 26
 constexpr float kC1 = 0.01f * 0.01f;
 constexpr float kC2 = 0.03f * 0.03f;
 
+// Tiles of a launch (256 threads each, fewer than 2^32 in all).
+constexpr int64_t kMaxTiles = 1ll << 24;
+
 struct LossLayout {
     size_t partial_off, dmaps_off, total;
     int64_t blocks;
@@ -69,9 +72,9 @@ static StripShape strip_shape(int64_t B, int64_t H, int64_t W, int64_t C) {
 }
 
 // Pixels of up to four channels stream; wider ones (whose halo of 10 C values
-// would not fit) take the tiles.
+// would not fit) take the tiles.  A column's byte offset in its row has 32 bits.
 static bool streams(int64_t B, int64_t H, int64_t W, int64_t C) {
-    return C <= 4 && W * C < (1ll << 31) - 4096 && strip_shape(B, H, W, C).blocks() < (1ll << 31) && B < 65536;
+    return C <= 4 && W * C < (1ll << 30) - 4096 && strip_shape(B, H, W, C).blocks() < (1ll << 31) && B < 65536;
 }
 
 static LossLayout loss_layout(int64_t B, int64_t H, int64_t W, int64_t C) {
@@ -599,6 +602,7 @@ int ubs_image_loss_fwd(int64_t B, int64_t H, int64_t W, int64_t C, const float *
     }
     const dim3 grid((unsigned)tiles, (unsigned)(B * C));
     const GaussWin win = gauss_window();
+    UBS_REQUIRE((ssim && streams(B, H, W, C)) || tiles < kMaxTiles, "image too large");
     if (ssim && streams(B, H, W, C)) {
         const StripShape s = strip_shape(B, H, W, C);
         const dim3 g((unsigned)s.blocks(), (unsigned)B);
@@ -653,6 +657,7 @@ int ubs_image_loss_bwd(int64_t B, int64_t H, int64_t W, int64_t C, const float *
     }
     const dim3 grid((unsigned)tiles, (unsigned)(B * C));
     const GaussWin win = gauss_window();
+    UBS_REQUIRE((lambda_dssim > 0.f && streams(B, H, W, C)) || tiles < kMaxTiles, "image too large");
     if (lambda_dssim > 0.f && streams(B, H, W, C)) {
         const StripShape s = strip_shape(B, H, W, C);
         const dim3 g((unsigned)s.blocks(), (unsigned)B);
