@@ -49,7 +49,6 @@ constexpr uint32_t kPairGroups = 16;                  // groups of 64 pairs of a
 constexpr uint32_t kPairPatches = 32;                 // patches whose bits it writes together
 constexpr uint32_t kTaskWords = 4;                    // groups of a task per thread of count (of kThreads), at most
 constexpr uint32_t kMaxPatches = 512;
-constexpr uint32_t kTaskPairs = 896;                  // pairs of a task aimed at: a window, with room for uneven blocks
 // Workgroups of count and place (fewer where there are fewer tasks): more than are
 // resident, so that what is left over at the end is small.
 constexpr uint32_t kCountBlocks = 2048, kPlaceBlocks = 4096;
@@ -70,7 +69,7 @@ static bool bin_shape(uint32_t C, uint32_t N, uint32_t tw, uint32_t th, BinShape
     if ((uint64_t)s.px * s.py > kMaxPatches) return false;
     s.patches = s.px * s.py;
     s.groups = (uint32_t)((total + 64 * kPairGroups - 1) / (64 * kPairGroups)) * kPairGroups;
-    s.most = std::max(std::min(1024u, 2 * s.groups + 64), s.groups / 200);
+    s.most = bins_most_tasks(s.groups / kPairGroups);
     s.bins = (uint64_t)tw * rows;
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     s.bits = up((size_t)total * sizeof(uint4));
@@ -190,8 +189,7 @@ __global__ __launch_bounds__(kCutThreads) void bins_cuts_kernel(uint32_t blocks,
         at += q < wave ? s_wave[q] : 0u;
         total += s_wave[q];
     }
-    const uint32_t aim = max(kTaskPairs, (uint32_t)(2 * (uint64_t)total / most) + 1);
-    const uint32_t floor = aim / 60 + 1;
+    const uint32_t aim = bins_task_aim(total, most), floor = bins_block_floor(aim);
     at += floor * g0;
     uint32_t k = at / aim;
     for (uint32_t g = g0; g < g1; g += U) {

@@ -431,6 +431,7 @@ def isect_finish(S: IsectState, n_isects: int, packed: int):
         # status the host has not read yet
         _call("ubs_isect_bins_place", C, S.N, tw, th, ptr(S.offsets), ptr(S.bins), S.bins.numel(), ptr(isect_ids),
               ptr(flatten_ids), n_isects, st)
+        S.bins = None  # (not held until the batch's other groups are placed)
         return S.tpg, isect_ids, flatten_ids, S.offsets
     if n_isects and S.order is not None:
         S.cum = torch.empty((C * S.N,), dtype=torch.int64, device=dev)
