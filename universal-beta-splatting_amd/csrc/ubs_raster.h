@@ -213,8 +213,10 @@ static __global__ __launch_bounds__(kOrderThreads) void raster_block_order_kerne
 __device__ __forceinline__ void support_box(float a, float b, float c, float &hx, float &hy) {
     const float det = a * c - b * b;
     if (det > 0.f) {
-        // (hardware reciprocal and square root, 1 ulp each: far inside the padding)
-        const float inv = __builtin_amdgcn_rcpf(det);
+        // (hardware reciprocal and square root, 1 ulp each: far inside the padding.
+        // Past 2^126 the reciprocal is a denormal, which it gives as 0: a smaller
+        // determinant widens the box)
+        const float inv = __builtin_amdgcn_rcpf(__builtin_amdgcn_fmed3f(det, 0.f, 0x1p126f));
         hx = __builtin_amdgcn_sqrtf(c * inv) * 1.001f + 1e-3f;
         hy = __builtin_amdgcn_sqrtf(a * inv) * 1.001f + 1e-3f;
     } else {
