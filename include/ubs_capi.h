@@ -348,8 +348,10 @@ int ubs_isect_tiles_emit_ordered_rec(uint32_t C, uint32_t N, const void *pair_re
  * bits, for visible depths without the sign bit (a negative depth's
  * sign-extended bits cover the id's upper half).
  *   ubs_isect_bins_workspace_bytes: 0 where the grid is past the method's
- *     limits (more than 65535 tile columns or camera rows, or 256 patches of
- *     32 x 32 tiles);
+ *     limits (more than 65535 tile columns or camera rows, or 512 patches of
+ *     32 columns x 16 rows, the cameras' rows stacked);
+ *   ubs_isect_bins_pays: whether it is faster than the sort for these sizes: 1, 0,
+ *     or, with n_isects -1 (not known yet), 2 where that depends on it;
  *   ubs_isect_bins_plan: pair_records from ubs_isect_tiles_count_info, order =
  *     the flat ids sorted by depth; writes the workspace and tile_offsets int32
  *     [C, th, tw] (as ubs_isect_offset_encode of the list);
@@ -357,6 +359,7 @@ int ubs_isect_tiles_emit_ordered_rec(uint32_t C, uint32_t N, const void *pair_re
  *     workspace and offsets.  Entries past n_isects are not stored.
  * No counterpart in the reference (it sorts all entries, isect_tiles.cu:224-278). */
 size_t ubs_isect_bins_workspace_bytes(uint32_t C, uint32_t N, uint32_t tile_width, uint32_t tile_height);
+int ubs_isect_bins_pays(uint32_t C, uint32_t N, uint32_t tile_width, uint32_t tile_height, int64_t n_isects);
 int ubs_isect_bins_plan(uint32_t C, uint32_t N, const void *pair_records, const int32_t *order,
                         uint32_t tile_size, uint32_t tile_width, uint32_t tile_height, int32_t *tile_offsets,
                         void *workspace, size_t workspace_bytes, void *stream);

@@ -71,3 +71,34 @@ def test_workspace_follows_the_pairs():
     assert size(1, 10_000, 512, 513) == 0 and size(1, 10_000, 513, 512) == 0  # 513 rows or columns: a patch more
     assert size(2, 10_000, 512, 256) > 0 and size(2, 10_000, 512, 257) == 0
     assert size(1, 10_000, 65536, 1) == 0
+
+
+def test_the_placement_is_taken_where_it_is_faster():
+    """The rule at sizes measured on both ways (us placed / sorted beside them)."""
+    from gsplat.cuda._backend import lib
+
+    pays = lib().ubs_isect_bins_pays
+    for C, N, tw, th, n, want in (
+            (1, 1_000_000, 120, 68, 5_783_480, 1),     # 267 / 399
+            (1, 1_000_000, 120, 68, 57_081, 1),        # 221 / 251
+            (2, 1_000_000, 120, 68, 117_066, 1),       # 292 / 296
+            (4, 1_000_000, 120, 68, 23_131_325, 1),    # 819 / 1084
+            (4, 1_000_000, 120, 68, 230_382, 0),       # 492 / 443
+            (8, 1_000_000, 120, 68, 46_244_700, 1),    # 1834 / 2295
+            (8, 1_000_000, 120, 68, 461_549, 0),       # 1028 / 746
+            (8, 100_000, 120, 68, 4_623_075, 1),       # 381 / 420
+            (8, 100_000, 120, 68, 46_389, 0),          # 319 / 255
+            (2, 1_000_000, 240, 135, 11_639_522, 1),   # 608 / 714
+            (2, 1_000_000, 240, 135, 115_285, 0),      # 425 / 312
+            (1, 10_000, 512, 512, 58_877, 0),          # 530 / 214
+            (1, 10_000, 512, 512, 616, 1),             # 530 / 1303
+            (1, 1_000_000, 512, 512, 5_853_432, 0),    # 872 / 465
+            (1, 1_000_000, 256, 256, 5_832_977, 1),    # 410 / 460
+            (1, 1_000_000, 1, 1, 1_000_000, 0),        # 430 / 249
+            (1, 100_000, 2, 2, 274_376, 0),            # 211 / 182
+            (1, 1_000_000, 8, 8, 4_968_502, 1),        # 272 / 326
+            (1, 1_000_000, 120, 68, 0, 1)):
+        assert pays(C, N, tw, th, n) == want, (C, N, tw, th, n)
+        assert pays(C, N, tw, th, -1) in (want, 2)
+    assert pays(1, 1_000_000, 120, 68, -1) == 1 and pays(1, 1_000_000, 512, 512, -1) == 2
+    assert pays(1, 1_000_000, 512, 513, 10 ** 9) == 0 and pays(1, 0, 120, 68, 0) == 0  # past the limits, no pairs

@@ -43,4 +43,28 @@ __host__ __device__ inline uint32_t bins_most_tasks(uint32_t blocks) {
     return few > many ? few : many;
 }
 
+// Whether placing the entries beats emitting and sorting them: 1 yes, 0 no, or,
+// with n_isects unknown (-1), 2: it depends on it.  Measured on both ways, us (1 to 8
+// cameras of 10k to 1M pairs, 1 x 1 to 512 x 512 tiles, all to 1% of them visible):
+//   - the sort moves an entry five times, 15 a million entries; its offset search
+//     runs over the tiles between two entries, 2.9 for every tile per entry; its
+//     launches 52 in all;
+//   - the placement looks at every patch for every pair and at its tiles one
+//     patch after another: 0.72 a patch and 0.21 a patch and million pairs.
+// 512 x 512 tiles (512 patches), 1M pairs, 5.9M entries: placed 872, sorted 465; 8
+// views of 1080p (136 patches), 8M pairs, 0.46M entries 1028 and 746, 46M entries 1834
+// and 2295; 616 entries on 512 x 512 tiles 530 and 1303.
+// A tile's entries of a window are stored by 16 lanes, so few tiles leave the chip
+// idle (1 x 1 tiles, 1M pairs: 430 placed, 249 sorted; 2 x 2: 331 and 282; 4 x 4 and
+// 100k: 188 and 182; 8 x 8: 177 and 187).
+constexpr uint32_t kPlaceMinTiles = 32;
+inline int bins_pays(uint64_t pairs, uint64_t tiles, uint32_t patches, int64_t n_isects) {
+    if (tiles < kPlaceMinTiles) return 0;
+    const double place = patches * (0.72 + 0.21e-6 * (double)pairs);
+    if (place <= 52.0) return 1;
+    if (n_isects < 0) return 2;
+    const double n = n_isects > 0 ? (double)n_isects : 1.0;
+    return place <= 52.0 + 15e-6 * n + 2.9 * (double)tiles / n;
+}
+
 }  // namespace ubs

@@ -587,6 +587,11 @@ size_t ubs_isect_bins_workspace_bytes(uint32_t C, uint32_t N, uint32_t tw, uint3
     return bin_shape(C, N, tw, th, s) ? s.bytes : 0;
 }
 
+int ubs_isect_bins_pays(uint32_t C, uint32_t N, uint32_t tw, uint32_t th, int64_t n_isects) {
+    BinShape s;
+    return bin_shape(C, N, tw, th, s) ? bins_pays((uint64_t)C * N, s.bins, s.patches, n_isects) : 0;
+}
+
 static int bins_check(uint32_t C, uint32_t N, uint32_t tw, uint32_t th, const void *ws, size_t ws_bytes, BinShape &s) {
     UBS_REQUIRE(bin_shape(C, N, tw, th, s), "tile grid or pair count past the direct placement's limits");
     UBS_REQUIRE(bit_width_u32(tw * th) + bit_width_u32(C) <= 32, "camera and tile ids need more than 32 bits");

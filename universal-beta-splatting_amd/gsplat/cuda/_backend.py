@@ -78,6 +78,7 @@ _SIGNATURES = {
     "ubs_isect_tiles_emit_ordered_rec": (
         _c_int, [_c_u32, _c_u32, _vp, _vp, _vp, _c_u32, _c_u32, _c_u32, _vp, _vp, _c_i64, _vp]),
     "ubs_isect_bins_workspace_bytes": (_c_size, [_c_u32, _c_u32, _c_u32, _c_u32]),
+    "ubs_isect_bins_pays": (_c_int, [_c_u32, _c_u32, _c_u32, _c_u32, _c_i64]),
     "ubs_isect_bins_plan": (_c_int, [_c_u32, _c_u32, _vp, _vp, _c_u32, _c_u32, _c_u32, _vp, _vp, _c_size, _vp]),
     "ubs_isect_bins_place": (_c_int, [_c_u32, _c_u32, _c_u32, _c_u32, _vp, _vp, _c_size, _vp, _vp, _c_i64, _vp]),
     "ubs_radix_sort_pairs_skip": (

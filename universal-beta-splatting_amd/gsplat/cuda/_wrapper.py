@@ -268,7 +268,9 @@ def isect_tiles(
     """Tiles per primitive [C,N] int32, isect ids int64 [n] (cam | tile |
     depth bits) sorted stably on their low 32 + tile_bits + cam_bits bits, and
     flatten ids int32 [n].  reference: _wrapper.py:285-343, isect_tiles.cu:99-285"""
-    return isect_tiles_offsets(means2d, radii, depths, tile_size, tile_width, tile_height, sort)[:3]
+    state = isect_begin(means2d, radii, depths, tile_size, tile_width, tile_height, sort)
+    (n_isects, packed), = isect_read_info([state])
+    return isect_finish(state, n_isects, packed, offsets=False)[:3]
 
 
 _SORT_MODES = ("depth_first", "segmented", "onesweep")
@@ -280,9 +282,10 @@ def set_isect_sort_mode(mode: str) -> None:
     ids and values, bit for bit:
       depth_first (default): the (camera, primitive) pairs sorted by depth
         once, then every entry stored at its place in the list (tile by tile,
-        in that order); with a negative visible depth, or a tile grid past
-        that method's limits, entries emitted in that order, then two
-        onesweep passes over the camera/tile bits;
+        in that order); with a negative visible depth, a tile grid past
+        that method's limits, or sizes it is slower for (under 32 tiles, or
+        many patches of tiles for few entries), entries emitted in that
+        order, then two onesweep passes over the camera/tile bits;
       segmented: entries in primitive order, onesweep over the camera/tile
         bits, then a per-tile depth sort in LDS;
       onesweep: onesweep passes over every byte of the ids."""
@@ -350,7 +353,7 @@ def isect_read_info(states) -> list:
 class IsectState:
     """The intersection stage up to the host read of n_isects (see isect_begin)."""
     __slots__ = ("means2d", "radii", "depths", "tile_size", "tile_width", "tile_height", "sort", "tpg", "cum",
-                 "info", "info_host", "ready", "order", "prec", "bins", "offsets", "C", "N")
+                 "info", "info_host", "ready", "order", "prec", "bins", "offsets", "pays", "C", "N")
 
 
 def isect_begin(means2d: Tensor, radii: Tensor, depths: Tensor, tile_size: int, tile_width: int, tile_height: int,
@@ -401,6 +404,7 @@ def isect_begin(means2d: Tensor, radii: Tensor, depths: Tensor, tile_size: int, 
               tile_height, ptr(S.tpg), ptr(S.cum), ptr(S.info), ptr(_late_status(dev)), None, None, None, ptr(ws),
               ws_bytes, st)
     S.order = S.info_host = S.ready = S.bins = S.offsets = None
+    S.pays = None  # whether the entries are placed (0: sorted, 2: with many patches it depends on n_isects)
     if depth_first:
         # the info leaves for the host first; the depth sort and what follows
         # from it run during the round trip
@@ -409,23 +413,34 @@ def isect_begin(means2d: Tensor, radii: Tensor, depths: Tensor, tile_size: int, 
         S.ready = torch.cuda.Event()
         S.ready.record(torch.cuda.current_stream(dev))
         _, S.order = radix_sort_pairs(dkeys, dvals, 0, 32, status_out=_late_status(dev))
-        bins_bytes = int(L.ubs_isect_bins_workspace_bytes(C, N, tile_width, tile_height))
-        if bins_bytes:
-            S.bins = torch.empty((bins_bytes,), dtype=torch.uint8, device=dev)
-            S.offsets = torch.empty((C, tile_height, tile_width), dtype=torch.int32, device=dev)
-            _call("ubs_isect_bins_plan", C, N, ptr(S.prec), ptr(S.order), tile_size, tile_width, tile_height,
-                  ptr(S.offsets), ptr(S.bins), bins_bytes, st)
+        if L.ubs_isect_bins_workspace_bytes(C, N, tile_width, tile_height):  # (0: past the placement's limits)
+            S.pays = L.ubs_isect_bins_pays(C, N, tile_width, tile_height, -1)
+            if S.pays == 1:
+                _plan_bins(S)
     return S
 
 
-def isect_finish(S: IsectState, n_isects: int, packed: int):
+def _plan_bins(S: IsectState) -> None:
+    """Queue the plan of the placement of the state's entries."""
+    C, N, tw, th, dev = S.C, S.N, S.tile_width, S.tile_height, S.means2d.device
+    bins_bytes = int(lib().ubs_isect_bins_workspace_bytes(C, N, tw, th))
+    S.bins = torch.empty((bins_bytes,), dtype=torch.uint8, device=dev)
+    S.offsets = torch.empty((C, th, tw), dtype=torch.int32, device=dev)
+    _call("ubs_isect_bins_plan", C, N, ptr(S.prec), ptr(S.order), S.tile_size, tw, th, ptr(S.offsets), ptr(S.bins),
+          bins_bytes, stream_of(S.means2d))
+
+
+def isect_finish(S: IsectState, n_isects: int, packed: int, offsets: bool = True):
     """Second half of isect_tiles, given the state's host-read info:
-    (tiles_per_gauss, isect_ids, flatten_ids, isect_offsets or None)."""
+    (tiles_per_gauss, isect_ids, flatten_ids, isect_offsets or None: where
+    offsets is False, or the sort does not give them)."""
     L = lib()
     C, dev, st = S.C, S.means2d.device, stream_of(S.means2d)
     tw, th, ts = S.tile_width, S.tile_height, S.tile_size
     isect_ids = torch.empty((n_isects,), dtype=torch.int64, device=dev)
     flatten_ids = torch.empty((n_isects,), dtype=torch.int32, device=dev)
+    if S.pays == 2 and packed >= 0 and L.ubs_isect_bins_pays(C, S.N, tw, th, n_isects):
+        _plan_bins(S)
     if S.bins is not None and packed >= 0:  # (a negative depth's bits cover the tile in the ids: sorted below)
         # capped at n_isects: the depth order may come from a sort whose
         # status the host has not read yet
@@ -444,7 +459,7 @@ def isect_finish(S: IsectState, n_isects: int, packed: int):
     elif n_isects:
         _call("ubs_isect_tiles_emit", C, S.N, ptr(S.means2d), ptr(S.radii), ptr(S.depths), ptr(S.cum), ts, tw, th,
               ptr(isect_ids), ptr(flatten_ids), st)
-    offsets = None
+    offs = None
     if n_isects and S.sort:
         end_bit = 32 + int(L.ubs_isect_prefix_bits(C, tw, th))
         late = _late_status(dev)
@@ -453,14 +468,16 @@ def isect_finish(S: IsectState, n_isects: int, packed: int):
         elif _sort_mode == "segmented":
             # stable on the camera/tile bits, then per tile on the depth bits
             ids1, flat1 = radix_sort_pairs(isect_ids, flatten_ids, 32, end_bit, status_out=late)
-            offsets = isect_offset_encode(ids1, C, tw, th)
+            offs = isect_offset_encode(ids1, C, tw, th)
             isect_ids, flatten_ids = torch.empty_like(ids1), torch.empty_like(flat1)
             _call("ubs_sort_tile_segments", n_isects, ptr(ids1), ptr(flat1), ptr(isect_ids), ptr(flatten_ids),
-                  ptr(offsets), C, tw, th, constant_depth_passes(packed), st)
+                  ptr(offs), C, tw, th, constant_depth_passes(packed), st)
         else:
             isect_ids, flatten_ids = radix_sort_pairs(isect_ids, flatten_ids, 0, end_bit,
                                                       skip_passes=constant_depth_passes(packed), status_out=late)
-    return S.tpg, isect_ids, flatten_ids, offsets
+    if offsets and S.pays is not None and packed >= 0:  # (the placement would have given them)
+        offs = isect_offset_encode(isect_ids, C, tw, th)
+    return S.tpg, isect_ids, flatten_ids, offs
 
 
 def constant_depth_passes(packed_range: int) -> int:
