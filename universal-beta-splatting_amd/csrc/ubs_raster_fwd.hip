@@ -182,8 +182,10 @@ __global__ __launch_bounds__(TS *TS) void raster_fwd_kernel(
             // 0.999 clamp), ordinary (finite values, 0 <= alpha, and no sigma that
             // underflows to -0: dx is 0 or at least 2^-25), or only by the general
             // code
+            // (as bits: one comparison for 0 <= v < 1e30)
+            const uint32_t large = __float_as_uint(1e30f);
             const bool ordinary =
-                op >= 0.f && op < 1e30f && be >= 0.f && be < 1e30f && ca >= 1e-12f && cc >= 1e-12f;
+                __float_as_uint(op) < large && __float_as_uint(be) < large && ca >= 1e-12f && cc >= 1e-12f;
             const bool plain = ordinary && op <= kNoClampOpacity;
             staged_mask = sub_mask | (ordinary ? 0u : kGeneralBit) | (plain ? 0u : kClampBit);
             if (entry_masks && write_meta) {  // for the backward
