@@ -58,10 +58,14 @@ struct StripShape {
 };
 
 // Longer strips repeat less of their halo (4 chunks: 44 input rows for 34 output
-// rows, 2: 22 for 12), shorter ones fill the chip: the longest that leave nearly
-// three workgroups for each of 256 CUs (1080p, three channels: 4 chunks, 736
-// workgroups, forward and backward 66 + 54 us; 6 chunks, 460: 64 + 58; 5, 552:
-// 81 + 64).
+// rows, 2: 22 for 12), shorter ones fill the chip.  512 workgroups of the forward
+// and 768 of the backward are resident, and a few past a multiple of either take
+// another round, so the time is not monotone in the length (1080p, three
+// channels, forward and backward with the host's calls, by chunks: 2, 2070
+// workgroups: 162 us; 3, 1081: 149; 4, 736: 127; 5, 552: 147; 6, 460: 134; 8,
+// 322: 165).  The longest with 700 workgroups or more is the best of them there and
+// within 20% of the best at every size measured from 256x256 to 3840x2160 (720p: 91
+// us with 2 chunks, 76 with 3; 2560x1440: 238 with 8, 208 with 7).
 static StripShape strip_shape(int64_t B, int64_t H, int64_t W, int64_t C) {
     StripShape s{};
     s.cols = (W * C + kStripCols - 1) / kStripCols;

@@ -6,16 +6,10 @@
 namespace ubs {
 
 // Beta kernel weight (1 - sigma)^beta with the hardware log2/exp2
-// (v_log_f32 / v_exp_f32).  The forward and the backward call this same
-// function, so the backward recovers transmittance from bit-identical alphas.
+// (v_log_f32 / v_exp_f32), as the forward takes it (the backward forms it from
+// (1 - sigma)^(beta - 1), which it needs as well).
 __device__ __forceinline__ float beta_pow(float one_minus_sigma, float beta) {
     return __builtin_amdgcn_exp2f(beta * __builtin_amdgcn_logf(one_minus_sigma));
-}
-
-// sigma = (a dx^2 + c dy^2) + 2b dx dy, the reference's grouping
-// (rasterize_to_pixels_fwd.cu:146-148); b2 = 2 b is exact.
-__device__ __forceinline__ float beta_sigma(float a, float b2, float c, float dx, float dy) {
-    return (a * dx * dx + c * dy * dy) + b2 * dx * dy;
 }
 
 // Workgroup -> (camera, tile).  Workgroups are dispatched round-robin over
@@ -254,20 +248,15 @@ __host__ __device__ __forceinline__ uint32_t subblock_mask(float mx, float my, f
 // a 1-D quadratic minimised in closed form and clamped to the edge.  The
 // threshold carries a margin of 1e-3 plus 1e-5 of the largest absolute term
 // sum over the rectangle, far above the rounding of the per-pixel fp32
-// sigma, so a pixel whose sigma the blend would accept is never culled.
-__host__ __device__ inline bool ellipse_meets_rect(float mx, float my, float a, float b, float c, float lo_x,
-                                                   float hi_x, float lo_y, float hi_y) {
+// sigma, so a pixel whose sigma the blend would accept is never culled.  (On
+// the host: the yardstick of subblock_mask_exact, which took its place.)
+inline bool ellipse_meets_rect(float mx, float my, float a, float b, float c, float lo_x, float hi_x, float lo_y,
+                               float hi_y) {
     const float dx0 = mx - hi_x, dx1 = mx - lo_x;  // offsets mean - pixel over the rectangle
     const float dy0 = my - hi_y, dy1 = my - lo_y;
     if (dx0 <= 0.f && dx1 >= 0.f && dy0 <= 0.f && dy1 >= 0.f) return true;
     if (!(a > 0.f && c > 0.f)) return true;
-#ifdef __HIP_DEVICE_COMPILE__
-    // only where on the edge the minimum is taken: 1 ulp there moves it by far
-    // less than the margin below
-    const float ia = __builtin_amdgcn_rcpf(a), ic = __builtin_amdgcn_rcpf(c);
-#else
     const float ia = 1.f / a, ic = 1.f / c;
-#endif
     float best = __builtin_huge_valf();
 #pragma unroll
     for (int e = 0; e < 2; ++e) {

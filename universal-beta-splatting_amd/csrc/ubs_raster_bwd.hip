@@ -12,10 +12,13 @@
 //   * A pixel's transmittance before each primitive is the state left by the
 //     groups behind it times the inclusive product over the row of
 //     1 / (1 - alpha), and the colour behind it the exclusive sum of
-//     alpha T (c . v): two 16-lane scans of four DPP steps each.  The forward
-//     and backward evaluate alpha with the same expressions, so the divisors
-//     are bit-identical; the recovery starts from the exact T after the last
-//     contributor (kept by the forward).
+//     alpha T (c . v): two 16-lane scans of four DPP steps each.  The
+//     recovery starts from the exact T after the last contributor (kept by the
+//     forward) and divides by this kernel's 1 - alpha.  sigma has the forward's
+//     bits; alpha = o (1 - sigma)^(beta - 1) (1 - sigma) here and
+//     o (1 - sigma)^beta there agree to about (3 + beta |log2(1 - sigma)|) 2^-23
+//     relative, and each primitive passed moves T by that times
+//     alpha / (1 - alpha).
 //   * A primitive's gradients (rasterize_to_pixels_bwd.cu:200-247) add up in
 //     its own lane's registers over the steps; the four rows are summed once
 //     per group (two permlane levels), turned through LDS so that 16
